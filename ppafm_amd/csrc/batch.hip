@@ -71,6 +71,7 @@ struct ppafm_batch {
 
     std::vector<long long> grid_off, pos_off, df_off, atom_off, brick_prefix;
     std::vector<BatchGridItem> gitems;
+    bool ortho_grids = true;  // every grid has orthogonal cell axes
     std::vector<DfGroup> groups;
 
     void *grids = nullptr;
@@ -159,10 +160,8 @@ bool homogeneous(const std::vector<BatchRelaxItem> &it)
 
 int enqueue_grid(ppafm_batch &b, int nitems, long long nbricks)
 {
-    bool ortho = true;
-    for (const BatchGridItem &g : b.gitems) ortho = ortho && ortho_cell(g.dcell);
     return launch_ff_build_batch(b.model, nitems, b.d_gitems, b.d_bprefix, nbricks, b.atoms, b.grids, b.f64,
-                                 b.any_uncharged, ortho, b.st);
+                                 b.any_uncharged, b.ortho_grids, b.st);
 }
 
 int enqueue_relax(ppafm_batch &b, const ppafm_batch_tuning &t, const BatchRelaxItem *items, const long long *prefix,
@@ -378,7 +377,6 @@ int build_plan(ppafm_batch *b, int nitems, const ppafm_batch_item *items)
         b->pos_off[k + 1] = b->pos_off[k] + npos;
         b->df_off[k + 1] = b->df_off[k] + (nzout > 0 ? (long long)s.scan.nx * s.scan.ny * nzout : 0);
         b->atom_off[k + 1] = b->atom_off[k] + s.natoms;
-        b->brick_prefix[k + 1] = b->brick_prefix[k] + ff_bricks(s.n);
         BatchGridItem &g = b->gitems[k];
         std::memset(&g, 0, sizeof(g));
         GridGeom gg = make_geom(s.n, s.cell);
@@ -387,7 +385,10 @@ int build_plan(ppafm_batch *b, int nitems, const ppafm_batch_item *items)
         g.atom_off = b->atom_off[k];
         g.grid_off = b->grid_off[k];
         for (int a = 0; a < 9; a++) g.dcell[a] = gg.dcell[a];
+        b->ortho_grids = b->ortho_grids && ortho_cell(g.dcell);
     }
+    for (int k = 0; k < nitems; k++)
+        b->brick_prefix[k + 1] = b->brick_prefix[k] + ff_bricks(items[k].n, b->model, b->f64, b->ortho_grids);
     PP_REQUIRE(b->brick_prefix[nitems] < (1LL << 31), "batch has too many grid bricks for one launch");
     // df groups: runs of equal nz among items with nz >= nw
     if (nw > 0) {

@@ -549,8 +549,9 @@ int launch_ff_build(const GridGeom &g, const ppafm_ff_model &m, int natoms, cons
     return dispatch(m, A, z0, atoms_dev, out, f64, nullptr, st);
 }
 
-long long ff_bricks(const int n[3])
+long long ff_bricks(const int n[3], const ppafm_ff_model &m, bool f64, bool ortho)
 {
+    if (!f64 && !(m.fp64_radius > 0) && ortho) return ff_boxes(n);
     return (long long)((n[0] + kColsX - 1) / kColsX) * ((n[1] + kColsY - 1) / kColsY) * ((n[2] + kZBrick - 1) / kZBrick);
 }
 

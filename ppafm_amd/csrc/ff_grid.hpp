@@ -126,4 +126,7 @@ struct BatchLaunch {
 int launch_ff_f32(const FFArgs &A, bool z0, bool with_lj, bool with_energy, const AtomRec *atoms, void *out,
                   const BatchLaunch *batch, bool ortho, hipStream_t st);
 
+// Launch blocks of the FP32 kernel on a grid with orthogonal cell axes.
+long long ff_boxes(const int n[3]);
+
 }  // namespace pp

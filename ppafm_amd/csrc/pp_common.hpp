@@ -88,8 +88,9 @@ namespace pp {
 // Device grid (z fastest): float4 (f64 = false) or double4 (f64 = true).
 int launch_ff_build(const GridGeom &g, const ppafm_ff_model &m, int natoms, const AtomRec *atoms_dev, void *out,
                     bool f64, hipStream_t st);
-// Bricks of one grid (launch blocks of the grid kernels).
-long long ff_bricks(const int n[3]);
+// Bricks of one grid: launch blocks of the grid kernel that a batch of the
+// model takes (ortho: every grid of the batch has orthogonal cell axes).
+long long ff_bricks(const int n[3], const ppafm_ff_model &m, bool f64, bool ortho);
 // Every grid of a batch in one launch; prefix[k] = bricks of items < k.
 int launch_ff_build_batch(const ppafm_ff_model &m, int nitems, const BatchGridItem *items_dev,
                           const long long *prefix_dev, long long nbricks, const AtomRec *atoms_dev, void *grids,
