@@ -12,8 +12,7 @@
 //   * 32-bit grid indices, ProbeParticle or OpenCL semantics chosen at
 //     compile time, per-lane tip base so the loop touches few uniforms.
 // Lanes run independent state machines over (z step, iteration) and stage
-// their output records in LDS (Stage, relax_dev.hpp); an LDS-staged
-// lock-step variant (relax_lds_kernel) is kept as an option.
+// their output records in LDS (Stage, relax_dev.hpp).
 
 #include <cstdlib>
 
@@ -32,7 +31,7 @@ namespace {
 // starts, the Newton phase.  A column is done when s reaches nz.  The plain
 // and warm kernels, per tile or with lane refill, all run these functions,
 // so a column's results do not depend on the lane, wave or launch shape.
-template <typename T4>
+template <int NC>  // components sampled: 3 forces, and the energy in mode 1
 struct Column {
     Stroke c;
     long obase;  // output offset of the column's item (0: pre-offset outputs)
@@ -40,7 +39,7 @@ struct Column {
     Fire S;
     int s, it, itr;
     bool sample;  // mode 0: next gather is the output sample
-    CellCache<T4> cache;
+    CellCache<NC> cache;
     // warm starts: Newton iterate q, iterations taken and allowed, FIRE
     // iteration of the next Newton try; `opening` = the step's first Newton
     // run (its failure is a fallback); `check` = S.r is a Newton zero not yet
@@ -54,8 +53,8 @@ struct Column {
 
 // Step 0 of column (i, j) (nothing to do when !live).  pred: the column's
 // step-0 estimate (3 floats) or nullptr.
-template <typename T4, int MODE, bool WARM>
-__device__ __forceinline__ void column_init(const DevArgs &A, Column<T4> &C, int i, int j, bool live, long obase,
+template <int MODE, bool WARM, int NC>
+__device__ __forceinline__ void column_init(const DevArgs &A, Column<NC> &C, int i, int j, bool live, long obase,
                                             const float *pred)
 {
     C.c = stroke_at(A, i, j);
@@ -69,7 +68,7 @@ __device__ __forceinline__ void column_init(const DevArgs &A, Column<T4> &C, int
     C.it = 0;
     C.itr = 0;
     C.sample = false;
-    C.cache.ix = C.cache.iy = C.cache.iz = -1;
+    clear_cell(C.cache);
     if (WARM) {
         C.next_try = A.newton_retry;
         C.qx = C.S.rx; C.qy = C.S.ry; C.qz = C.S.rz;
@@ -89,23 +88,36 @@ __device__ __forceinline__ void column_init(const DevArgs &A, Column<T4> &C, int
     }
 }
 
-// One force evaluation of a plain column: FIRE to convergence at each z
-// step, outputs in stroke order.  Counts force evaluations and finished
-// positions.
+// Shares of a wave's running lanes that wait before it turns to them (serve):
+// plain FIRE, ProbeParticle and OpenCL semantics, and warm starts.  Measured
+// from one lane (at once) down to half the wave: 256x256x60 scan 8.8 ms at
+// once, 6.6 at 1/16, 6.4 at 1/8, 7.2 at 1/4; 48 molecules of 128x128x30 plain
+// 16.1, 13.1, 12.9, 16.9; Newton 6.4 ms at once, 5.6 at 1/8, 5.2 at 1/4, 5.1
+// at 1/2; 400x400x60 tilted scan 3.3, 2.7, 2.6, 2.8.
+constexpr int kServe[2] = {8, 4};
+constexpr int kServeWarm = 4;
+
+// One pass of a plain column, a force evaluation unless the lane waits: FIRE
+// to convergence at each z step, outputs in stroke order.  Counts force
+// evaluations and finished positions.
 // BUF: grid loads through a buffer resource (orthogonal kernels whose
 // lanes share one grid); the lanes of a refill wave may each read another
 // grid, and a buffer resource per lane would be a loop over the lanes'
 // distinct grids at every load, so they use plain global loads.
-template <typename T4, int MODE, int K, bool ORTHO = false, bool BUF = ORTHO>
-__device__ __forceinline__ void column_step(const DevArgs &A, const T4 *__restrict__ grid, Column<T4> &C, Stage<K> &G,
+template <typename T4, int MODE, int K, bool ORTHO, bool BUF, int FRAC, int NC>
+__device__ __forceinline__ void column_step(const DevArgs &A, const T4 *__restrict__ grid, Column<NC> &C, Stage<K> &G,
                                             unsigned long long &nevals, unsigned long long &npos)
 {
-    double fe[4], gx, gy, gz;
+    double fe[4], gx, gy, gz, ux, uy, uz;
     to_grid<ORTHO>(A, C.S.rx, C.S.ry, C.S.rz, gx, gy, gz);
     // the orthogonal kernels also read the grid through a buffer resource
     // (the host picks them for grids under 4 GiB only)
-    gather_cached<T4, BUF, MODE == 1>(grid, A, gx, gy, gz, fe, C.cache);
-    nevals++;
+    if (MODE == 0) {
+        const bool due = serve<FRAC>(C.sample);
+        if (C.sample && !due) return;
+    }
+    if (!cell_cached<T4, BUF, FRAC>(grid, A, gx, gy, gz, C.cache, ux, uy, uz)) return;
+    cell_force(C.cache, ux, uy, uz, fe);
     bool done = false;
     const long o = C.obase + C.c.col0 + C.s;
     if (MODE == 0 && C.sample) {
@@ -128,6 +140,7 @@ __device__ __forceinline__ void column_step(const DevArgs &A, const T4 *__restri
         }
     }
     if (done) {
+        nevals += C.it + (MODE == 0 ? 1 : 0);  // a move each, and mode 0's output sample
         npos++;
         C.s++;
         if (C.s < A.nz) {
@@ -138,7 +151,7 @@ __device__ __forceinline__ void column_step(const DevArgs &A, const T4 *__restri
     }
 }
 
-// One force evaluation of a warm-started column.  Every step begins with
+// One pass of a warm-started column.  Every step begins with
 // Newton iterations on the interpolated field (newton_from) from the
 // continuation start the reference uses (step 0: from the column's estimate,
 // or the plain start without one; with newton_extrap2 > 0, steps >= 2 from
@@ -164,29 +177,28 @@ __device__ __forceinline__ void column_step(const DevArgs &A, const T4 *__restri
 // the next step continues from FIRE's result.  Newton iterates and FIRE
 // moves share the cell cache of the corners (a load only when the cell
 // changes); Newton evaluations count in nevals.
-template <typename T4, int MODE, int K, bool ORTHO = false, bool BUF = ORTHO>
-__device__ __forceinline__ void column_step_warm(const DevArgs &A, const T4 *__restrict__ grid, Column<T4> &C,
+template <typename T4, int MODE, int K, bool ORTHO, bool BUF, int NC>
+__device__ __forceinline__ void column_step_warm(const DevArgs &A, const T4 *__restrict__ grid, Column<NC> &C,
                                                  Stage<K> &G, unsigned long long &nevals, unsigned long long &npos,
                                                  unsigned long long &nfb)
 {
     double gx, gy, gz, ux, uy, uz;
     to_grid<ORTHO>(A, C.newton ? C.qx : C.S.rx, C.newton ? C.qy : C.S.ry, C.newton ? C.qz : C.S.rz, gx, gy, gz);
     // the cell cache: Newton iterates near convergence and FIRE's moves mostly stay in one cell
-    corners_cached<T4, BUF, MODE == 1>(grid, A, gx, gy, gz, C.cache, ux, uy, uz);
-    const T4 *v = C.cache.v;
+    if (!cell_cached<T4, BUF, kServeWarm>(grid, A, gx, gy, gz, C.cache, ux, uy, uz)) return;
     nevals++;
     bool done = false;
     const long o = C.obase + C.c.col0 + C.s;
     const bool retry = !C.newton && !(MODE == 0 && C.sample) && A.newton_retry > 0 && C.it >= C.next_try;
     bool fire = !C.newton;
     double fe[4];
-    interp8(v, ux, uy, uz, fe, MODE == 1);
+    cell_force(C.cache, ux, uy, uz, fe);
     if (C.newton || retry) {
         double px = C.newton ? C.qx : C.S.rx, py = C.newton ? C.qy : C.S.ry, pz = C.newton ? C.qz : C.S.rz;
         bool stable;
         double st2, f2;
         const bool ok =
-            newton_from<T4, MODE, ORTHO>(A, v, ux, uy, uz, fe, C.tx, C.ty, C.tz, px, py, pz, A.newton_cap, stable, st2, f2) &&
+            newton_from<MODE, ORTHO>(A, C.cache, ux, uy, uz, fe, C.tx, C.ty, C.tz, px, py, pz, A.newton_cap, stable, st2, f2) &&
             stable;
         if (retry) C.next_try = C.it + A.newton_retry;
         const bool gated = C.gate && !(f2 <= A.ws_res2);
@@ -284,24 +296,25 @@ __device__ __forceinline__ void column_step_warm(const DevArgs &A, const T4 *__r
     }
 }
 
-// One pixel column (i, j) from start to end.
-template <typename T4, int MODE, int K, bool ORTHO = false>
+// One pixel column (i, j) from start to end; turns: the loop passes it took.
+template <typename T4, int MODE, int K, bool ORTHO, int FRAC>
 __device__ __forceinline__ void relax_column(const DevArgs &A, const T4 *__restrict__ grid, int i, int j, bool live,
-                                             Stage<K> &G, unsigned long long &nevals, unsigned long long &npos)
+                                             Stage<K> &G, unsigned long long &nevals, unsigned long long &npos,
+                                             unsigned &turns)
 {
-    Column<T4> C;
-    column_init<T4, MODE, false>(A, C, i, j, live, 0, nullptr);
-    while (C.s < A.nz) column_step<T4, MODE, K, ORTHO>(A, grid, C, G, nevals, npos);
+    Column<MODE == 1 ? 4 : 3> C;
+    column_init<MODE, false>(A, C, i, j, live, 0, nullptr);
+    for (; C.s < A.nz; turns++) column_step<T4, MODE, K, ORTHO, ORTHO, FRAC>(A, grid, C, G, nevals, npos);
 }
 
 template <typename T4, int MODE, int K, bool ORTHO = false>
 __device__ __forceinline__ void relax_column_warm(const DevArgs &A, const T4 *__restrict__ grid, int i, int j,
                                                   bool live, Stage<K> &G, unsigned long long &nevals,
-                                                  unsigned long long &npos, unsigned long long &nfb)
+                                                  unsigned long long &npos, unsigned long long &nfb, unsigned &turns)
 {
-    Column<T4> C;
-    column_init<T4, MODE, true>(A, C, i, j, live, 0, A.pred ? A.pred + 3 * ((long)i * A.ny + j) : nullptr);
-    while (C.s < A.nz) column_step_warm<T4, MODE, K, ORTHO>(A, grid, C, G, nevals, npos, nfb);
+    Column<MODE == 1 ? 4 : 3> C;
+    column_init<MODE, true>(A, C, i, j, live, 0, A.pred ? A.pred + 3 * ((long)i * A.ny + j) : nullptr);
+    for (; C.s < A.nz; turns++) column_step_warm<T4, MODE, K, ORTHO, ORTHO>(A, grid, C, G, nevals, npos, nfb);
 }
 
 // Wave sum of the per-lane counters, one atomic per wave.  `passes` (the
@@ -337,28 +350,27 @@ constexpr int stage_batch()
     return WARM ? 4 : 1;
 }
 
-// WPB waves (tiles) per workgroup.  Block b runs WPB consecutive tiles of
-// part b % 8 (one contiguous part of the tiles per XCD).
-template <typename T4, int MODE, bool ORTHO, int WPB>
+// A wave relaxes a tile of A.tile_x x A.tile_y columns (64 or fewer, its
+// remaining lanes idle).  Block b runs its waves' consecutive tiles of part
+// b % 8 (one contiguous part of the tiles per XCD).
+// FRAC 0 in tiles of a few columns, where lanes seldom wait together.
+template <typename T4, int MODE, bool ORTHO, int WPB, int FRAC>
 __global__ __launch_bounds__(64 * WPB) void relax_dev_kernel(DevArgs A, const T4 *__restrict__ grid)
 {
-    __shared__ __align__(16) unsigned char lds[kStageSingle * 64 * WPB * kStageRecordBytes];
-    Stage<kStageSingle> G = make_stage<kStageSingle>(lds, 64 * WPB, threadIdx.x);
+    extern __shared__ __align__(16) unsigned char single_lds[];  // kStageSingle records per column
+    const int wave = WPB == 1 ? 0 : (int)(threadIdx.x / 64);
+    const int lane = WPB == 1 ? (int)threadIdx.x : (int)(threadIdx.x % 64);
+    const int cols = A.tile_x * A.tile_y;
     const int per_xcd = ((A.ntiles + WPB - 1) / WPB + 7) / 8;
     const int b = blockIdx.x;
-    int tile, lane;
-    if constexpr (WPB == 1) {
-        tile = (b % 8) * per_xcd + b / 8;
-        lane = threadIdx.x;
-    } else {
-        tile = ((b % 8) * per_xcd + b / 8) * WPB + (int)(threadIdx.x / 64);
-        lane = threadIdx.x % 64;
-    }
+    const int tile = ((b % 8) * per_xcd + b / 8) * WPB + wave;
     if (tile >= A.ntiles) return;
+    Stage<kStageSingle> G = make_stage<kStageSingle>(single_lds, cols * WPB, wave * cols + min(lane, cols - 1));
     const int ti = tile / A.tiles_y, tj = tile % A.tiles_y;
-    const int i = ti * 8 + lane / 8, j = tj * 8 + lane % 8;
+    const int i = ti * A.tile_x + lane / A.tile_y, j = tj * A.tile_y + lane % A.tile_y;
     unsigned long long nevals = 0, npos = 0;
-    relax_column<T4, MODE, kStageSingle, ORTHO>(A, grid, i, j, i < A.nx && j < A.ny, G, nevals, npos);
+    unsigned turns = 0;
+    relax_column<T4, MODE, kStageSingle, ORTHO, FRAC>(A, grid, i, j, lane < cols && i < A.nx && j < A.ny, G, nevals, npos, turns);
     flush_counters(A.counters, nevals, npos, lane);
 }
 
@@ -439,15 +451,15 @@ __global__ __launch_bounds__(256) void relax_batch_kernel(DevArgs A0, BatchArgs 
             const int lt = (int)(tile - prefix[m]);
             const int ti = lt / it.tiles_y, tj = lt % it.tiles_y;
             const int i = ti * TX + lane / TY, j = tj * TY + lane % TY;
-            const unsigned long long before = nevals;
+            unsigned turns = 0;
             if (WARM)
                 relax_column_warm<T4, MODE, KS, ORTHO>(A, grids + it.grid_off, i, j, i < A.nx && j < A.ny, G, nevals, npos,
-                                                       nfb);
-            else relax_column<T4, MODE, KS, ORTHO>(A, grids + it.grid_off, i, j, i < A.nx && j < A.ny, G, nevals, npos);
-            // the tile's loop passes: every pass evaluates once in each lane still running
-            unsigned long long d = nevals - before;
-            for (int off = 32; off > 0; off >>= 1) d = max(d, (unsigned long long)__shfl_xor(d, off, 64));
-            passes += d;
+                                                       nfb, turns);
+            else
+                relax_column<T4, MODE, KS, ORTHO, kServe[MODE]>(A, grids + it.grid_off, i, j, i < A.nx && j < A.ny, G, nevals,
+                                                                npos, turns);
+            for (int off = 32; off > 0; off >>= 1) turns = max(turns, (unsigned)__shfl_xor(turns, off, 64));
+            passes += turns;
         }
     }
     flush_counters(A0.counters, nevals, npos, lane, nfb, WARM, passes, true);
@@ -479,7 +491,7 @@ __global__ __launch_bounds__(256) void relax_refill_kernel(DevArgs A, BatchArgs 
     const long long ncols = (long long)B.nitems * cols_item;
     const long long per = (ncols + 7) / 8;
     unsigned long long nevals = 0, npos = 0, nfb = 0, passes = 0;
-    Column<T4> C;
+    Column<MODE == 1 ? 4 : 3> C;
     C.s = A.nz;  // no column yet
     const T4 *grid = grids;
     int q = 0;         // parts of the column range this wave found empty (uniform)
@@ -529,7 +541,7 @@ __global__ __launch_bounds__(256) void relax_refill_kernel(DevArgs A, BatchArgs 
                     grid = grids + it.grid_off;
                     const float *pred =
                         WARM && B.pred ? B.pred + 3 * ((long long)it.col_off + (long long)i * A.ny + j) : nullptr;
-                    column_init<T4, MODE, WARM>(A, C, i, j, live, it.out_off, pred);
+                    column_init<MODE, WARM>(A, C, i, j, live, it.out_off, pred);
                     need = false;  // a column outside the scan (live false) is done at once
                 }
             }
@@ -543,163 +555,11 @@ __global__ __launch_bounds__(256) void relax_refill_kernel(DevArgs A, BatchArgs 
         }
         if (C.s < A.nz) {
             if (WARM) column_step_warm<T4, MODE, KS, ORTHO, false>(A, grid, C, G, nevals, npos, nfb);
-            else column_step<T4, MODE, KS, ORTHO, false>(A, grid, C, G, nevals, npos);
+            else column_step<T4, MODE, KS, ORTHO, false, kServe[MODE]>(A, grid, C, G, nevals, npos);
         }
         passes++;
     }
     flush_counters(A.counters, nevals, npos, lane, nfb, WARM, passes, true);
-}
-
-// ---------------------------------------------------------------------------
-// LDS-staged variant.  The lanes of a wave relax z step s together; before
-// the step the wave reduces its probes' bounding box (grid index space),
-// copies that block of the grid (plus a margin) into LDS as structure-of-
-// arrays planes, and every gather whose 8 corners fall inside the block
-// reads LDS; the others read global memory.  The per-lane arithmetic is the
-// shared helpers', so the results equal relax_dev_kernel's.
-constexpr int kMargin = 2;
-
-template <typename T>
-__device__ __forceinline__ T wave_min(T v)
-{
-    for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-    return v;
-}
-template <typename T>
-__device__ __forceinline__ T wave_max(T v)
-{
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
-__device__ __forceinline__ int wrapi(int i, int n)
-{
-    i %= n;
-    return i < 0 ? i + n : i;
-}
-
-template <typename T4, int MODE>
-__global__ __launch_bounds__(64) void relax_lds_kernel(DevArgs A, const T4 *__restrict__ grid, int cap)
-{
-    using T = decltype(T4::x);
-    extern __shared__ __align__(16) unsigned char smem[];
-    T *LX = (T *)smem;
-    T *LY = LX + cap;
-    T *LZ = LY + cap;
-    T *LW = LZ + cap;  // energy plane, mode 1 only (cap counts 4 planes then)
-
-    const int per_xcd = (A.ntiles + 7) / 8;
-    const int b = blockIdx.x;
-    const int tile = (b % 8) * per_xcd + b / 8;
-    if (tile >= A.ntiles) return;  // uniform per block
-    const int ti = tile / A.tiles_y, tj = tile % A.tiles_y;
-    const int lane = threadIdx.x;
-    const int i = ti * 8 + lane / 8, j = tj * 8 + lane % 8;
-    const bool live = i < A.nx && j < A.ny;
-    const int nz = A.nz;
-    const Stroke c = stroke_at(A, i, j);
-    double tx, ty, tz;
-    tip_pos(A, c, 0, live, tx, ty, tz);
-    double ox, oy, oz;
-    probe_offset<MODE>(A, ox, oy, oz);
-    Fire S{tx + ox, ty + oy, tz + oz, 0, 0, 0, A.dtmax, A.a0};
-    unsigned long long nevals = 0, npos = 0;
-
-    for (int s = 0; s < nz; s++) {
-        if (s > 0) next_step<MODE>(A, c, s, live, tx, ty, tz, S);
-        // ---- stage the block around the wave's probes
-        double g0x, g0y, g0z;
-        to_grid(A, S.rx, S.ry, S.rz, g0x, g0y, g0z);
-        const float big = 3.0e38f;
-        const float mnx = wave_min(live ? (float)g0x : big), mxx = wave_max(live ? (float)g0x : -big);
-        const float mny = wave_min(live ? (float)g0y : big), mxy = wave_max(live ? (float)g0y : -big);
-        const float mnz = wave_min(live ? (float)g0z : big), mxz = wave_max(live ? (float)g0z : -big);
-        // block only when all bounds are finite and small (a diverging probe
-        // sends its wave to global memory instead)
-        const bool sane = mnx > -1.0e7f && mxx < 1.0e7f && mny > -1.0e7f && mxy < 1.0e7f && mnz > -1.0e7f && mxz < 1.0e7f &&
-                          mxx - mnx < 512.f && mxy - mny < 512.f && mxz - mnz < 512.f;
-        int lox = 0, loy = 0, loz = 0, ex = 0, ey = 0, ez = 0;
-        if (sane) {
-            lox = (int)floorf(mnx) - kMargin; loy = (int)floorf(mny) - kMargin; loz = (int)floorf(mnz) - kMargin;
-            ex = (int)floorf(mxx) + 1 + kMargin - lox + 1;
-            ey = (int)floorf(mxy) + 1 + kMargin - loy + 1;
-            ez = (int)floorf(mxz) + 1 + kMargin - loz + 1;
-        }
-        const bool staged = sane && (long)ex * ey * ez <= cap;
-        if (staged) {
-            const int vol = ex * ey * ez;
-            for (int q = lane; q < vol; q += 64) {
-                const int cz = q % ez, t = q / ez;
-                const int bb = t % ey, a = t / ey;
-                const unsigned gi = ((unsigned)wrapi(lox + a, A.n0) * A.n1 + wrapi(loy + bb, A.n1)) * A.n2 + wrapi(loz + cz, A.n2);
-                const T4 v = grid[gi];
-                LX[q] = v.x; LY[q] = v.y; LZ[q] = v.z;
-                if (MODE == 1) LW[q] = v.w;
-            }
-        }
-        __syncthreads();
-
-        // ---- relax this step, all lanes together
-        int st = live ? 0 : 2;  // 0 = FIRE, 1 = output sample pending (mode 0), 2 = done
-        int it = 0, itr = 0;
-        bool capped = false;
-        float4 outf = make_float4(0.f, 0.f, 0.f, 0.f);
-        while (__ballot(st < 2) != 0) {
-            if (st < 2) {
-                double gx, gy, gz;
-                to_grid(A, S.rx, S.ry, S.rz, gx, gy, gz);
-                const double flx = floor(gx), fly = floor(gy), flz = floor(gz);
-                double fe[4];
-                // inside test in floating point (false for NaN), before any int conversion
-                if (staged && flx >= lox && flx + 1 < lox + ex && fly >= loy && fly + 1 < loy + ey && flz >= loz &&
-                    flz + 1 < loz + ez) {
-                    const int a = (int)flx - lox, bb = (int)fly - loy, cz = (int)flz - loz;
-                    const int q00 = (a * ey + bb) * ez + cz, q01 = q00 + ez, q10 = q00 + ey * ez, q11 = q10 + ez;
-                    const int q[8] = {q00, q00 + 1, q01, q01 + 1, q10, q10 + 1, q11, q11 + 1};
-                    T4 v[8];
-#pragma unroll
-                    for (int k = 0; k < 8; k++) {
-                        v[k].x = LX[q[k]]; v[k].y = LY[q[k]]; v[k].z = LZ[q[k]];
-                        v[k].w = MODE == 1 ? LW[q[k]] : (T)0;
-                    }
-                    interp8(v, gx - flx, gy - fly, gz - flz, fe, MODE == 1);
-                } else {
-                    gather(grid, A, gx, gy, gz, fe, MODE == 1);
-                }
-                nevals++;
-                if (MODE == 0 && st == 1) {
-                    outf = make_float4((float)fe[0], (float)fe[1], (float)fe[2], 0.f);
-                    st = 2;
-                } else {
-                    const double ff = fire_move<MODE>(A, fe, tx, ty, tz, S);
-                    it++;
-                    const bool conv = ff < A.conv_f2;
-                    if (conv || it >= A.max_iters) {
-                        capped = !conv;
-                        if (MODE == 0) {
-                            itr = conv ? it - 1 : A.max_iters;
-                            st = 1;
-                        } else {
-                            outf = tip_frame_force(A, fe);
-                            itr = it;
-                            st = 2;
-                        }
-                    }
-                }
-            }
-        }
-        if (live) {
-            const long o = c.col0 + s;
-            store_pos(A, o, S.rx, S.ry, S.rz);
-            if (A.force) A.force[o] = outf;
-            if (A.iters) A.iters[o] = itr;
-            const double fo[4] = {outf.x, outf.y, outf.z, 0.0};
-            store_status(A, o, capped, S.rx, S.ry, S.rz, fo);
-            npos++;
-        }
-        __syncthreads();
-    }
-    flush_counters(A.counters, nevals, npos, lane);
 }
 
 }  // namespace
@@ -718,33 +578,56 @@ static int simd_count()
     return 4 * cus;
 }
 
-// Single-scan launch.  With one-wave workgroups the dispatcher has been
-// seen to place two waves of this launch on one SIMD while another SIMD of
-// the CU idles, depending on what ran before it (c1, 1024 tiles, right after
-// its grid build: 8.9-9.3 ms, against 7.1-7.4 ms after another FIRE launch).
-// A scan with more than 3 tiles per CU and at most one per SIMD (c1)
-// therefore uses four-wave workgroups, one per CU with its waves on the
-// CU's four SIMDs.  Smaller scans keep one-wave workgroups spread over the
-// CUs (four-wave workgroups there leave CUs idle: a 256-tile scan 3.80 ->
-// 4.07 ms; two-wave workgroups on 512 tiles ran 1 % slower), and so do
-// scans beyond one tile per SIMD, which LDS lets 6 to a CU.
-template <typename T4, int MODE, bool ORTHO, int WPB>
+// Single-scan launch.  A column's steps are a serial chain, so a scan takes
+// as long as its slowest wave, and a wave is faster the fewer columns it holds
+// (its lanes reach new cells and step ends at different passes).  Tiles are
+// therefore as small as the SIMDs allow, one wave each: the smallest power of
+// two of columns that leaves no more tiles than SIMDs, 4 at least (2 and 1 run
+// the same or slower) and 64 at most.  Relaxation alone, 64 columns a wave
+// against this: 24x24x20 scan (4 columns) 1.75 -> 1.54 ms, 128x128x40 (16)
+// 2.89 -> 2.73, 128x128x30 OpenCL semantics (16) 0.86 -> 0.70; half as many
+// columns again, two waves on a SIMD, is slower: 128x128x40 (8) 4.98,
+// 256x256x60 (32 against 64) 8.15 against 6.17.
+// With one-wave workgroups the dispatcher has been seen to place two waves of
+// such a launch on one SIMD while another SIMD of the CU idles, depending on
+// what ran before it (256x256x60: 8.9-9.3 ms against 7.1-7.4; 128x128x40 3.65
+// against 2.65).  A scan with more than 3 tiles per CU and at most one per
+// SIMD uses four-wave workgroups, one per CU with its waves on the CU's four
+// SIMDs.  Others keep one-wave workgroups spread over the CUs (four-wave
+// workgroups there leave CUs idle), and so do scans beyond one tile per SIMD.
+template <typename T4, int MODE, bool ORTHO, int WPB, int FRAC>
 static void launch_single_w(const DevArgs &A, const void *grid, hipStream_t st)
 {
     const long nb = (((A.ntiles + WPB - 1L) / WPB + 7) / 8) * 8;
-    hipLaunchKernelGGL((relax_dev_kernel<T4, MODE, ORTHO, WPB>), dim3((unsigned)nb), dim3(64 * WPB), 0, st, A,
+    const size_t lds = (size_t)A.tile_x * A.tile_y * WPB * kStageSingle * kStageRecordBytes;
+    hipLaunchKernelGGL((relax_dev_kernel<T4, MODE, ORTHO, WPB, FRAC>), dim3((unsigned)nb), dim3(64 * WPB), lds, st, A,
                        (const T4 *)grid);
 }
 
 template <typename T4, int MODE, bool ORTHO>
-static void launch_single(const DevArgs &A, const void *grid, hipStream_t st)
+static void launch_single(const DevArgs &A0, const void *grid, hipStream_t st)
 {
     const int simds = simd_count();
     const int cus = simds / 4;
-    if (cus > 0 && A.ntiles > 3L * cus && A.ntiles <= simds) {
-        launch_single_w<T4, MODE, ORTHO, 4>(A, grid, st);
+    DevArgs A = A0;
+    static const int tiles[][2] = {{2, 2}, {4, 2}, {4, 4}, {8, 4}, {8, 8}};
+    for (const auto &t : tiles) {
+        A.tile_x = t[0];
+        A.tile_y = t[1];
+        A.tiles_y = (A.ny + t[1] - 1) / t[1];
+        const long n = ((A.nx + t[0] - 1L) / t[0]) * A.tiles_y;
+        if (n <= simds || t[0] * t[1] == 64) {
+            A.ntiles = (int)n;
+            break;
+        }
+    }
+    const bool wide = A.tile_x * A.tile_y >= 16;
+    if (wide && cus > 0 && A.ntiles > 3L * cus && A.ntiles <= simds) {
+        launch_single_w<T4, MODE, ORTHO, 4, kServe[MODE]>(A, grid, st);
+    } else if (wide) {
+        launch_single_w<T4, MODE, ORTHO, 1, kServe[MODE]>(A, grid, st);
     } else {
-        launch_single_w<T4, MODE, ORTHO, 1>(A, grid, st);
+        launch_single_w<T4, MODE, ORTHO, 1, 0>(A, grid, st);
     }
 }
 
@@ -758,8 +641,6 @@ int launch_relax_fast(const RelaxLaunch &L, const void *grid, bool f64, hipStrea
     DevArgs A;
     A.n0 = L.g.n[0]; A.n1 = L.g.n[1]; A.n2 = L.g.n[2];
     A.nx = L.scan.nx; A.ny = L.scan.ny; A.nz = L.scan.nz;
-    A.tiles_y = (A.ny + 7) / 8;
-    A.ntiles = ((A.nx + 7) / 8) * A.tiles_y;
     A.max_iters = L.rp.max_iters;
     A.probe_start = L.rp.probe_start;
     for (int k = 0; k < 9; k++) { A.dinv[k] = L.g.dinv[k]; A.rot[k] = L.tip.rot[k]; }
@@ -775,31 +656,8 @@ int launch_relax_fast(const RelaxLaunch &L, const void *grid, bool f64, hipStrea
     A.pos = L.out.pos; A.pos_f32 = L.out.pos_f32; A.force = (float4 *)L.out.force; A.iters = L.out.iters;
     A.status = L.out.status;
     A.counters = L.out.counters;
-    if (A.ntiles == 0 || A.nz == 0) return 0;
-    const long nblk = ((A.ntiles + 7L) / 8) * 8;
-    PP_REQUIRE(nblk < (1L << 31), "scan too large");
-    dim3 grd((unsigned)nblk), blk(64);
-    // LDS-staged lock-step kernel: off unless PPAFM_RELAX_LDS_KB > 0 (38 KB
-    // lets 4 waves share a CU's 160 KB).  Lock-step makes a wave wait for its
-    // slowest lane at every z step; on the 120-atom scan that lengthens the
-    // slowest wave's chain from 10,411 to 23,650 evaluations, more than the
-    // ~30% per-evaluation gain of LDS gathers buys back.
-    static const char *lds_env = getenv("PPAFM_RELAX_LDS_KB");
-    const int lds_kb = lds_env ? atoi(lds_env) : 0;
-    if (lds_kb > 0) {
-        const int esz = f64 ? 8 : 4;
-        const int planes = L.rp.mode == 1 ? 4 : 3;
-        const int cap = (lds_kb * 1024) / (planes * esz);
-        const size_t bytes = (size_t)cap * planes * esz;
-        if (f64) {
-            if (L.rp.mode == 0) hipLaunchKernelGGL((relax_lds_kernel<double4, 0>), grd, blk, bytes, st, A, (const double4 *)grid, cap);
-            else hipLaunchKernelGGL((relax_lds_kernel<double4, 1>), grd, blk, bytes, st, A, (const double4 *)grid, cap);
-        } else {
-            if (L.rp.mode == 0) hipLaunchKernelGGL((relax_lds_kernel<float4, 0>), grd, blk, bytes, st, A, (const float4 *)grid, cap);
-            else hipLaunchKernelGGL((relax_lds_kernel<float4, 1>), grd, blk, bytes, st, A, (const float4 *)grid, cap);
-        }
-        return 0;
-    }
+    if (A.nx == 0 || A.ny == 0 || A.nz == 0) return 0;
+    PP_REQUIRE((A.nx + 7L) / 8 * ((A.ny + 7L) / 8) < (1L << 31) - 8, "scan too large");
     // orthogonal cell axes (every configuration here): the diagonal of dinv
     // alone, and grid reads through a buffer resource (32-bit offsets: the
     // grid under 4 GiB)

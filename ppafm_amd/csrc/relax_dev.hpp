@@ -15,6 +15,7 @@ namespace {
 struct DevArgs {
     int n0, n1, n2;
     int nx, ny, nz;
+    int tile_x, tile_y;  // columns of a wave's tile (single scans)
     int tiles_y, ntiles;
     int max_iters;
     int probe_start;
@@ -120,15 +121,46 @@ __device__ __forceinline__ void corners(const T4 *__restrict__ g, const DevArgs 
     v[4] = g[c10 + iz]; v[5] = g[c10 + jz]; v[6] = g[c11 + iz]; v[7] = g[c11 + jz];
 }
 
-// The 8 corners of the cell a probe last sampled, kept in registers across
-// its FIRE iterations: while the probe stays in that cell (most iterations
-// of a converging step) the sample needs no memory access.  The values are
-// the grid's, so results equal those of gather().
-template <typename T4>
+// The cell a probe last sampled, kept in registers across its FIRE
+// iterations: while the probe stays in that cell (most iterations of a
+// converging step) the sample needs no memory access.  Kept is the cell's
+// trilinear polynomial
+//   F = c0 + c1 z + y (c2 + c3 z) + x (c4 + c5 z + y (c6 + c7 z))
+// in the position (x, y, z) within the cell, FP64: 7 FMAs per component where
+// the weighted sum of the corners takes 8 and 15 more for the weights (and,
+// on float4 grids, a conversion per corner).  NC components: force, and the
+// energy in mode 1.
+// (bx, by, bz): the cell's lower corner in grid coordinates, before the
+// periodic wrap.  A cell never sampled has NaN there, which is in no cell.
+template <int NC>
 struct CellCache {
-    int ix = -1, iy = -1, iz = -1;
-    T4 v[8];
+    double bx, by, bz;
+    double c[8][NC];
 };
+
+template <int NC>
+__device__ __forceinline__ void clear_cell(CellCache<NC> &C)
+{
+    C.bx = C.by = C.bz = __builtin_nan("");
+}
+
+// 0 <= u < 1, by the bits: the high word of such a number is below that of
+// 1.0; a sign bit, 1 and more, infinities and NaN are not
+__device__ __forceinline__ bool in_cell(double ux, double uy, double uz)
+{
+    const unsigned a = (unsigned)__double2hiint(ux), b = (unsigned)__double2hiint(uy), c = (unsigned)__double2hiint(uz);
+    return max(a, max(b, c)) < 0x3FF00000u;
+}
+
+template <int NC>
+__device__ __forceinline__ void cell_force(const CellCache<NC> &C, double ux, double uy, double uz, double out[4])
+{
+    out[3] = 0;
+#pragma unroll
+    for (int i = 0; i < NC; i++)
+        out[i] = fma(ux, fma(uy, fma(uz, C.c[7][i], C.c[6][i]), fma(uz, C.c[5][i], C.c[4][i])),
+                     fma(uy, fma(uz, C.c[3][i], C.c[2][i]), fma(uz, C.c[1][i], C.c[0][i])));
+}
 
 typedef double pp_d2 __attribute__((ext_vector_type(2)));
 typedef float pp_f4 __attribute__((ext_vector_type(4)));
@@ -155,45 +187,79 @@ __device__ __forceinline__ T4 buf_corner(__amdgpu_buffer_rsrc_t r, unsigned idx)
     }
 }
 
-// corners() through the cache: C.v holds the corners of the cell of
-// (gx, gy, gz) afterwards; (ux, uy, uz) is the position in it.  BUF: the
-// loads go through a buffer resource on g (buf_corner; the caller makes
-// sure the grid is under 4 GiB).
-template <typename T4, bool BUF = false, bool WANT_W = true>
-__device__ __forceinline__ void corners_cached(const T4 *__restrict__ g, const DevArgs &A, double gx, double gy,
-                                               double gz, CellCache<T4> &C, double &ux, double &uy, double &uz)
+// Whether the wave turns to the lanes that wait: at least 1/FRAC of its
+// running lanes do.  A wave's lanes reach a new cell, or the end of a step, at
+// different passes of their loop; a wave that follows each lane at once runs
+// those blocks (some 100 instructions and a load's latency) on nearly every
+// pass for a few lanes.  A waiting lane repeats nothing and skips nothing, so
+// its results do not depend on when it is served.  FRAC 0: at once.
+template <int FRAC>
+__device__ __forceinline__ bool serve(bool waiting)
 {
-    int ix, jx, iy, jy, iz, jz;
-    axis(gx, A.n0, ix, jx, ux);
-    axis(gy, A.n1, iy, jy, uy);
-    axis(gz, A.n2, iz, jz, uz);
-    if (ix != C.ix || iy != C.iy || iz != C.iz) {
+    if (FRAC == 0) return true;
+    return FRAC * __popcll(__ballot(waiting)) >= __popcll(__ballot(true));
+}
+
+template <int NC, typename T4>
+__device__ __forceinline__ void corner_values(const T4 &v, double o[NC])
+{
+    o[0] = (double)v.x; o[1] = (double)v.y; o[2] = (double)v.z;
+    if constexpr (NC == 4) o[3] = (double)v.w;
+}
+
+// The cell of grid coordinates (gx, gy, gz) into C, loaded unless it is
+// there; (ux, uy, uz) is the position in it.  False: not there, and the lane
+// waits for others that need a load (serve<FRAC>).  BUF: the loads go through a
+// buffer resource on g (buf_corner; the caller makes sure the grid is under
+// 4 GiB).
+template <typename T4, bool BUF, int FRAC, int NC>
+__device__ __forceinline__ bool cell_cached(const T4 *__restrict__ g, const DevArgs &A, double gx, double gy, double gz,
+                                            CellCache<NC> &C, double &ux, double &uy, double &uz)
+{
+    ux = gx - C.bx;
+    uy = gy - C.by;
+    uz = gz - C.bz;
+    const bool hit = in_cell(ux, uy, uz);
+    const bool due = serve<FRAC>(!hit);
+    if (!hit && due) {
+        int ix, jx, iy, jy, iz, jz;
+        axis(gx, A.n0, ix, jx, ux);
+        axis(gy, A.n1, iy, jy, uy);
+        axis(gz, A.n2, iz, jz, uz);
+        C.bx = floor(gx);
+        C.by = floor(gy);
+        C.bz = floor(gz);
         const unsigned c00 = ((unsigned)ix * A.n1 + iy) * A.n2, c01 = ((unsigned)ix * A.n1 + jy) * A.n2;
         const unsigned c10 = ((unsigned)jx * A.n1 + iy) * A.n2, c11 = ((unsigned)jx * A.n1 + jy) * A.n2;
+        T4 v[8];
         if constexpr (BUF) {
             const __amdgpu_buffer_rsrc_t r =
                 __builtin_amdgcn_make_buffer_rsrc(const_cast<T4 *>(g), (short)0, (int)0xFFFFFFFF, 0x00020000);
-            C.v[0] = buf_corner<T4, WANT_W>(r, c00 + iz); C.v[1] = buf_corner<T4, WANT_W>(r, c00 + jz);
-            C.v[2] = buf_corner<T4, WANT_W>(r, c01 + iz); C.v[3] = buf_corner<T4, WANT_W>(r, c01 + jz);
-            C.v[4] = buf_corner<T4, WANT_W>(r, c10 + iz); C.v[5] = buf_corner<T4, WANT_W>(r, c10 + jz);
-            C.v[6] = buf_corner<T4, WANT_W>(r, c11 + iz); C.v[7] = buf_corner<T4, WANT_W>(r, c11 + jz);
+            v[0] = buf_corner<T4, NC == 4>(r, c00 + iz); v[1] = buf_corner<T4, NC == 4>(r, c00 + jz);
+            v[2] = buf_corner<T4, NC == 4>(r, c01 + iz); v[3] = buf_corner<T4, NC == 4>(r, c01 + jz);
+            v[4] = buf_corner<T4, NC == 4>(r, c10 + iz); v[5] = buf_corner<T4, NC == 4>(r, c10 + jz);
+            v[6] = buf_corner<T4, NC == 4>(r, c11 + iz); v[7] = buf_corner<T4, NC == 4>(r, c11 + jz);
         } else {
-            C.v[0] = g[c00 + iz]; C.v[1] = g[c00 + jz]; C.v[2] = g[c01 + iz]; C.v[3] = g[c01 + jz];
-            C.v[4] = g[c10 + iz]; C.v[5] = g[c10 + jz]; C.v[6] = g[c11 + iz]; C.v[7] = g[c11 + jz];
+            v[0] = g[c00 + iz]; v[1] = g[c00 + jz]; v[2] = g[c01 + iz]; v[3] = g[c01 + jz];
+            v[4] = g[c10 + iz]; v[5] = g[c10 + jz]; v[6] = g[c11 + iz]; v[7] = g[c11 + jz];
         }
-        C.ix = ix;
-        C.iy = iy;
-        C.iz = iz;
+        double d[8][NC];
+#pragma unroll
+        for (int k = 0; k < 8; k++) corner_values<NC>(v[k], d[k]);
+#pragma unroll
+        for (int i = 0; i < NC; i++) {
+            const double z0 = d[1][i] - d[0][i], z1 = d[3][i] - d[2][i], z2 = d[5][i] - d[4][i], z3 = d[7][i] - d[6][i];
+            C.c[0][i] = d[0][i];
+            C.c[1][i] = z0;
+            C.c[2][i] = d[2][i] - d[0][i];
+            C.c[3][i] = z1 - z0;
+            C.c[4][i] = d[4][i] - d[0][i];
+            C.c[5][i] = z2 - z0;
+            C.c[6][i] = (d[6][i] - d[4][i]) - C.c[2][i];
+            C.c[7][i] = (z3 - z2) - C.c[3][i];
+        }
     }
-}
-
-template <typename T4, bool BUF = false, bool WANT_E = true>
-__device__ __forceinline__ void gather_cached(const T4 *__restrict__ g, const DevArgs &A, double gx, double gy,
-                                              double gz, double out[4], CellCache<T4> &C)
-{
-    double ux, uy, uz;
-    corners_cached<T4, BUF, WANT_E>(g, A, gx, gy, gz, C, ux, uy, uz);
-    interp8(C.v, ux, uy, uz, out, WANT_E);
+    return hit || due;
 }
 
 template <typename T4>
@@ -285,8 +351,8 @@ __device__ __forceinline__ double fire_move(const DevArgs &A, const double fe[4]
 // One Newton step toward the zero of the total force on the trilinear grid
 // field: J dr = -F with the exact Jacobian of the interpolant in the current
 // cell (derivatives of the trilinear weights mapped by dinv) plus the
-// springs' Jacobian, from the cell's 8 corners v, the fractional position
-// (ux, uy, uz) of r in it and the grid force fe there (interp8), all FP64.
+// springs' Jacobian, from the cell's polynomial C, the fractional position
+// (ux, uy, uz) of r in it and the grid force fe there (cell_force), all FP64.
 // A step longer than max_step is cut to that length (damped Newton).
 // Returns false, leaving r unchanged, when the step is not finite; st2 =
 // squared length of the full step, f2 = squared total force at the old r.  `stable` tells whether the Jacobian at r
@@ -294,25 +360,19 @@ __device__ __forceinline__ double fire_move(const DevArgs &A, const double fe[4]
 // characteristic polynomial l^3 + a2 l^2 + a1 l + a0): only then is a zero of
 // the force there a minimum that damped dynamics settle in, not a saddle or a
 // maximum such as the point straight above a repulsive atom.
-template <typename T4, int MODE, bool ORTHO = false>
-__device__ __forceinline__ bool newton_from(const DevArgs &A, const T4 v[8], double ux, double uy, double uz,
+template <int MODE, bool ORTHO, int NC>
+__device__ __forceinline__ bool newton_from(const DevArgs &A, const CellCache<NC> &C, double ux, double uy, double uz,
                                             const double fe[4], double tx, double ty, double tz, double &rx,
                                             double &ry, double &rz, double max_step, bool &stable, double &st2,
                                             double &f2)
 {
-    double dT[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};  // dT[i][a] = dF_i / du_a
+    double dT[3][3];  // dT[i][a] = dF_i / du_a
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const int bx = k >> 2, by = (k >> 1) & 1, bz = k & 1;
-        const double wx = bx ? ux : 1 - ux, wy = by ? uy : 1 - uy, wz = bz ? uz : 1 - uz;
-        const double d0 = (bx ? 1.0 : -1.0) * wy * wz, d1 = wx * (by ? 1.0 : -1.0) * wz, d2 = wx * wy * (bz ? 1.0 : -1.0);
-        const double c[3] = {(double)v[k].x, (double)v[k].y, (double)v[k].z};
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-            dT[i][0] = fma(c[i], d0, dT[i][0]);
-            dT[i][1] = fma(c[i], d1, dT[i][1]);
-            dT[i][2] = fma(c[i], d2, dT[i][2]);
-        }
+    for (int i = 0; i < 3; i++) {
+        const double p = fma(uz, C.c[7][i], C.c[6][i]);  // d2F / dx dy
+        dT[i][0] = fma(uy, p, fma(uz, C.c[5][i], C.c[4][i]));
+        dT[i][1] = fma(ux, p, fma(uz, C.c[3][i], C.c[2][i]));
+        dT[i][2] = fma(ux, fma(uy, C.c[7][i], C.c[5][i]), fma(uy, C.c[3][i], C.c[1][i]));
     }
     double J[3][3];
 #pragma unroll
@@ -381,19 +441,6 @@ __device__ __forceinline__ bool newton_from(const DevArgs &A, const T4 v[8], dou
     return true;
 }
 
-template <typename T4, int MODE>
-__device__ __forceinline__ bool newton_step(const DevArgs &A, const T4 *__restrict__ g, double tx, double ty,
-                                            double tz, double &rx, double &ry, double &rz, double max_step,
-                                            bool &stable)
-{
-    double gx, gy, gz, ux, uy, uz, st2, f2, fe[4];
-    to_grid(A, rx, ry, rz, gx, gy, gz);
-    T4 v[8];
-    corners(g, A, gx, gy, gz, v, ux, uy, uz);
-    interp8(v, ux, uy, uz, fe, false);
-    return newton_from<T4, MODE>(A, v, ux, uy, uz, fe, tx, ty, tz, rx, ry, rz, max_step, stable, st2, f2);
-}
-
 __device__ __forceinline__ void store_pos(const DevArgs &A, long o, double rx, double ry, double rz)
 {
     if (!A.pos) return;
@@ -411,14 +458,6 @@ __device__ __forceinline__ void store_pos(const DevArgs &A, long o, double rx, d
 // never fire): bit 0 = the iteration cap ended the step without meeting the
 // stop rule, bit 1 = a non-finite position or grid force (a NaN grid or a
 // diverging probe); 0 = converged.
-__device__ __forceinline__ void store_status(const DevArgs &A, long o, bool capped, double rx, double ry, double rz,
-                                             const double fe[4])
-{
-    if (!A.status) return;
-    const bool finite = isfinite(rx) && isfinite(ry) && isfinite(rz) && isfinite(fe[0]) && isfinite(fe[1]) && isfinite(fe[2]);
-    A.status[o] = (unsigned char)((capped ? 1 : 0) | (finite ? 0 : 2));
-}
-
 __device__ __forceinline__ unsigned char status_byte(bool capped, double rx, double ry, double rz, const double fe[4])
 {
     const bool finite = isfinite(rx) && isfinite(ry) && isfinite(rz) && isfinite(fe[0]) && isfinite(fe[1]) && isfinite(fe[2]);
