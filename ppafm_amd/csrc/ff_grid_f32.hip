@@ -293,7 +293,7 @@ constexpr double kFarDist = 6.0;  // A
 // less than their pair sums; below it every atom of the box counts as near.
 constexpr int kFarMin = 12;
 constexpr int kBoxTile = kThreads;  // atoms per LDS tile, one per thread
-constexpr int kNearCap = 512;       // near atoms listed; beyond, every tile is staged for each slab
+constexpr int kNearCap = 512;       // near atoms listed; beyond, every atom is staged for each slab
 constexpr int kWPad = kP + 1;       // row stride against LDS bank conflicts
 
 // Chebyshev nodes on [-1, 1] and the values of their Lagrange polynomials at
@@ -336,6 +336,11 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
     const double ccx = dcx * cx, ccy = dcy * cy, ccz = dcz * cz;
     const double hx = half * fabs(dcx), hy = half * fabs(dcy), hz = half * fabs(dcz);
     const double dfar = fmax(kFarDist, kFarRatio * fmax(hx, fmax(hy, hz)));
+    auto is_far = [&](const AtomRec &a) {
+        const double rx = a.x - ccx, ry = a.y - ccy, rz = a.z - ccz;
+        const double ex = fmax(fabs(rx) - hx, 0.0), ey = fmax(fabs(ry) - hy, 0.0), ez = fmax(fabs(rz) - hz, 0.0);
+        return ex * ex + ey * ey + ez * ez >= dfar * dfar && isfinite(rx) && isfinite(ry) && isfinite(rz);
+    };
     for (int e = t; e < kBox * kP; e += kThreads) L.w[(e / kP) * kWPad + e % kP] = F.w[e];
 
     // ---- far atoms at the nodes.  128 lanes hold the nodes, 4 along z each;
@@ -360,13 +365,10 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
         for (int i0 = 0; i0 < A.natoms; i0 += kBoxTile) {
             const bool in = i0 + t < A.natoms;
             AtomRec a = {};
-            double rx = 0, ry = 0, rz = 0;
             bool far = false;
             if (in) {
                 a = atoms[i0 + t];
-                rx = a.x - ccx; ry = a.y - ccy; rz = a.z - ccz;
-                const double ex = fmax(fabs(rx) - hx, 0.0), ey = fmax(fabs(ry) - hy, 0.0), ez = fmax(fabs(rz) - hz, 0.0);
-                far = ex * ex + ey * ey + ez * ez >= dfar * dfar && isfinite(rx) && isfinite(ry) && isfinite(rz);
+                far = is_far(a);
             }
             const unsigned long long mf = __ballot(far), mn = __ballot(in && !far);
             if (lane == 0) {
@@ -388,7 +390,7 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
                 if (in && t < kNearCap) L.list[t] = t;
                 break;
             }
-            if (far) L.rec[pf + __popcll(mf & below)] = atom_record(a, rx, ry, rz);
+            if (far) L.rec[pf + __popcll(mf & below)] = atom_record(a, a.x - ccx, a.y - ccy, a.z - ccz);
             else if (in) {
                 const int p = pn + __popcll(mn & below);
                 if (p < kNearCap) L.list[p] = i0 + t;
@@ -422,15 +424,23 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
     }
     __syncthreads();
 
-    // ---- the points, in slabs of 4 x: a lane holds 4 z points of a column
-    const int col = t >> 2, zl = t & 3;
-    const int xi = col >> 4, y = col & 15;
+    // ---- the points, in slabs of 4 x: a wave holds 4x4 columns, a lane 4 z
+    // points of one.  Near pairs are summed in coordinates relative to the
+    // centre of the wave's columns (and of 64 points along z), which keeps the
+    // rounding of a point within 1e-8 A in x and y.
+    const int col = lane >> 2, zl = lane & 3;
+    const int xi = col >> 2, y = wave * 4 + (col & 3);
+    const int c2 = xi * kBox + y;  // the column's row in t2
     const int iy = by * kBox + y;
-    const double fy = iy - cy;
+    const double wcy = by * kBox + wave * 4 + 1.5, wcz = (bz * kBox / kZBrick) * kZBrick + 0.5 * (kZBrick - 1);
+    const double fy = iy - wcy;
+    const double oy = dcy * wcy, oz = dcz * wcz;
     for (int slab = 0; slab < kBox / 4; slab++) {
         if (bx * kBox + slab * 4 >= A.n[0]) break;  // uniform
         const int ix = bx * kBox + slab * 4 + xi;
-        const double fx = ix - cx;
+        const double wcx = bx * kBox + slab * 4 + 1.5;
+        const double fx = ix - wcx;
+        const double ox = dcx * wcx;
         double aL[kK][4], aE[kK][4];
 #pragma unroll
         for (int k = 0; k < kK; k++)
@@ -470,7 +480,7 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
 #pragma unroll 2
                 for (int q = 0; q < kP; q++) {
 #pragma unroll
-                    for (int c = 0; c < NG; c++) v[c] = L.t2[c][col * kWPad + q];
+                    for (int c = 0; c < NG; c++) v[c] = L.t2[c][c2 * kWPad + q];
 #pragma unroll
                     for (int k = 0; k < kK; k++) {
                         const double w = L.w[(zl + 4 * k) * kWPad + q];
@@ -489,36 +499,36 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
         for (int k = 0; k < kK; k++) {
             px[k] = (float)(dcx * fx);
             py[k] = (float)(dcy * fy);
-            pz[k] = (float)(dcz * ((zl + 4 * k) - half));
+            pz[k] = (float)(dcz * (bz * kBox + zl + 4 * k - wcz));
         }
         const bool listed = nnear <= kNearCap;
         const int total = listed ? nnear : A.natoms;
-        for (int i0 = 0; i0 < total; i0 += kBoxTile) {
-            const int nt = min(kBoxTile, total - i0);
-            if (t < nt) {
-                const AtomRec a = atoms[listed ? L.list[i0 + t] : i0 + t];
-                const double rx = a.x - ccx, ry = a.y - ccy, rz = a.z - ccz;
-                AtomLds r = atom_record(a, rx, ry, rz);
-                if (!listed && use_far) {  // a far atom is in the polynomial already: its terms here are zeros
-                    const double ex = fmax(fabs(rx) - hx, 0.0), ey = fmax(fabs(ry) - hy, 0.0), ez = fmax(fabs(rz) - hz, 0.0);
-                    if (ex * ex + ey * ey + ez * ez >= dfar * dfar && isfinite(rx) && isfinite(ry) && isfinite(rz)) {
-                        r.hi.w = 0.f;
-                        r.lj = make_float4(0.f, 0.f, 0.f, 0.f);
-                    }
+        AtomLds *rec = L.rec + wave * 64;  // each wave stages the atoms for itself
+        for (int i0 = 0; i0 < total; i0 += 64) {
+            const int nt = min(64, total - i0);
+            if (lane < nt) {
+                const AtomRec a = atoms[listed ? L.list[i0 + lane] : i0 + lane];
+                AtomLds r = atom_record(a, a.x - ox, a.y - oy, a.z - oz);
+                if (!listed && use_far && is_far(a)) {  // in the polynomial already: its terms here are zeros
+                    r.hi.w = 0.f;
+                    r.lj = make_float4(0.f, 0.f, 0.f, 0.f);
                 }
-                L.rec[t] = r;
+                rec[lane] = r;
             }
-            __syncthreads();
-            sum_f32<LJ, NS, Z0, WE, QS, true, SEP, true>(A, L.rec, 0, 1, nt, px, py, pz, kK, aL, aE);
-            __syncthreads();
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            sum_f32<LJ, NS, Z0, WE, QS, true, SEP, true>(A, rec, 0, 1, nt, px, py, pz, kK, aL, aE);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
+        __syncthreads();  // the next slab's t1, t2 share the records' memory
         if (ix < A.n[0] && iy < A.n[1]) {
 #pragma unroll
             for (int k = 0; k < kK; k++) {
                 const int iz = bz * kBox + zl + 4 * k;
                 if (iz >= A.n[2]) break;
                 out[((long)ix * A.n[1] + iy) * A.n[2] + iz] =
-                    point_value<LJ, NS, WE, SEP>(A, atoms, ccx + dcx * fx, ccy + dcy * fy, ccz + dcz * (iz - cz), aL[k], aE[k]);
+                    point_value<LJ, NS, WE, SEP>(A, atoms, ox + dcx * fx, oy + dcy * fy, oz + dcz * (iz - wcz), aL[k], aE[k]);
             }
         }
     }
