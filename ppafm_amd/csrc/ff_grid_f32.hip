@@ -44,12 +44,12 @@ namespace pp {
 
 namespace {
 
-// One atom against a lane's kK points (ALL: the first nk of them).  SEP:
+// One atom against a lane's K points (ALL: the first nk of them).  SEP:
 // separate LJ and Coulomb accumulators sL, sE (mode 0), else one, sL (mode 1).
 // ORTHO: the points share x and y (orthogonal cell axes).
-template <bool LJ, int NS, bool Z0, bool WE, bool QS, bool ORTHO, bool SEP, bool ALL>
+template <bool LJ, int NS, bool Z0, bool WE, bool QS, bool ORTHO, bool SEP, bool ALL, int K>
 __device__ __forceinline__ void atom_f32(const FFArgs &A, const AtomLds &a, const float *px, const float *py,
-                                         const float *pz, int nk, float sL[kK][4], float sE[kK][4])
+                                         const float *pz, int nk, float sL[K][4], float sE[K][4])
 {
     const float4 hi = a.hi;
     const float4 lo = a.lo;
@@ -63,7 +63,7 @@ __device__ __forceinline__ void atom_f32(const FFArgs &A, const AtomLds &a, cons
         dxy2 = __fmaf_rn(dx0, dx0, __fmaf_rn(dy0, dy0, A.r2safe));
     }
 #pragma unroll
-    for (int k = 0; k < kK; k++) {
+    for (int k = 0; k < K; k++) {
         if (!ALL && k >= nk) break;
         const float dx = ORTHO ? dx0 : (px[k] - hi.x) - lo.x;
         const float dy = ORTHO ? dy0 : (py[k] - hi.y) - lo.y;
@@ -139,21 +139,21 @@ __device__ __forceinline__ void atom_f32(const FFArgs &A, const AtomLds &a, cons
 
 // Sums over the atoms lds[first], lds[first + step], ... (n of them) at the
 // lane's points: FP32 partial sums of kFold atoms folded into FP64.
-template <bool LJ, int NS, bool Z0, bool WE, bool QS, bool ORTHO, bool SEP, bool ALL>
+template <bool LJ, int NS, bool Z0, bool WE, bool QS, bool ORTHO, bool SEP, bool ALL, int K = kK>
 __device__ __forceinline__ void sum_f32(const FFArgs &A, const AtomLds *lds, int first, int step, int n, const float *px,
-                                        const float *py, const float *pz, int nk, double aL[kK][4], double aE[kK][4])
+                                        const float *py, const float *pz, int nk, double aL[K][4], double aE[K][4])
 {
     for (int j0 = 0; j0 < n; j0 += kFold) {
         const int j1 = min(n, j0 + kFold);
-        float sL[kK][4], sE[kK][4];
+        float sL[K][4], sE[K][4];
 #pragma unroll
-        for (int k = 0; k < kK; k++)
+        for (int k = 0; k < K; k++)
 #pragma unroll
             for (int c = 0; c < 4; c++) { sL[k][c] = 0.f; sE[k][c] = 0.f; }
         for (int j = j0; j < j1; j++)
-            atom_f32<LJ, NS, Z0, WE, QS, ORTHO, SEP, ALL>(A, lds[first + j * step], px, py, pz, nk, sL, sE);
+            atom_f32<LJ, NS, Z0, WE, QS, ORTHO, SEP, ALL, K>(A, lds[first + j * step], px, py, pz, nk, sL, sE);
 #pragma unroll
-        for (int k = 0; k < kK; k++)
+        for (int k = 0; k < K; k++)
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 aL[k][c] += (double)sL[k][c];
@@ -270,25 +270,32 @@ __device__ __forceinline__ void brick_f32(const FFArgs &A, const AtomRec *__rest
 }
 
 // Orthogonal cells: a block computes a box of 16^3 points.  The field of an
-// atom farther from the box than kFarRatio half widths (and kFarDist) is
-// smooth over it, so far atoms are summed at the box's kP^3 Chebyshev nodes
-// only, and the sums are carried to the 4096 points by the nodes' tensor-
-// product polynomial in FP64; atoms nearer are summed at every point.  A far
-// pair costs 1/8 of a near one; VALU bound as before, in the near pairs for a
-// molecule, in the nodes for a slab.
-// Interpolation error: < 8e-8 of the far atoms' force for the shipped species
-// and tips at ratio 8 (0.1 A steps: 6 A), under the FP32 pair sums' own
-// rounding (4e-7 at the median point of a slab's grid, 2e-6 at the 99th
-// percentile, before and after).  Order 7 loses a digit (8e-7), and so do
-// ratios 6.7 and 6 (1.1e-6, 6e-7).  kFarDist keeps the steep r^-13 repulsion
-// out of the polynomial on grids finer than 0.1 A.
+// atom farther from the box than kFarRatio half widths, and so far that its
+// repulsion is below 1/24 of its attraction, is smooth over it: such far atoms
+// are summed at the box's kP^3 Chebyshev nodes only, and the sums are carried
+// to the 4096 points by the nodes' tensor-product polynomial in FP64; atoms
+// nearer are summed at every point.  A far pair costs 1/8 of a near one.  With
+// more atoms than one LDS tile, those beyond kVeryFarRatio half widths are
+// summed at kP2^3 nodes (1/33), whose polynomial is added to the values at the
+// kP^3 nodes.  VALU bound as before, in the near pairs for a molecule, in the
+// nodes for a slab.
+// Interpolation error, against the far atom's own force on 0.1 A steps: order
+// 8 at ratio 8 (6 A) 8e-8 for C, H, N, O and 5e-7 for Au at its 6.9 A; order 5
+// at ratio 40 (30 A) 3e-7 of the Lennard-Jones force, 5e-9 of the Coulomb
+// force.  The FP32 pair sums' own rounding is 4e-7 of the total at the median
+// point of a slab's grid and 2e-6 at the 99th percentile, before and after.
+// Order 7, or ratio 6.7, loses a digit at 6 A; order 4 at 30 A two.
 // Measured (grid kernel, before: every atom at every point): 60 atoms, dz2
 // tip, 256x256x192 points 1277 -> 373 us; 16 such grids of 8-120 atoms
-// 23.5 -> 6.6 ms; 17,928 atoms, 400x400x300 points 321 -> 43 ms.
+// 23.5 -> 6.6 ms; 17,928 atoms, 400x400x300 points 321 -> 43 ms with one set of
+// nodes, 14.7 ms with two.
 constexpr int kBox = 16;
 constexpr int kP = 8;
 constexpr double kFarRatio = 8.0;
-constexpr double kFarDist = 6.0;  // A
+constexpr double kFarForces = 24.0;  // attraction over repulsion
+constexpr int kP2 = 5;
+constexpr double kVeryFarRatio = 40.0;
+constexpr int kGroups = 10;  // lane groups of kP2^2 that share the atoms, kP2 nodes along z a lane
 // Far atoms a box needs before the polynomial (56 FP64 FMAs per point) costs
 // less than their pair sums; below it every atom of the box counts as near.
 constexpr int kFarMin = 12;
@@ -301,6 +308,8 @@ constexpr int kWPad = kP + 1;       // row stride against LDS bank conflicts
 struct FarTable {
     double x[kP];
     double w[kBox * kP];
+    double x2[kP2];
+    double w2[kP * kP2];  // the second set's polynomials at the first set's nodes
 };
 
 template <int NG>  // fields summed together: force, and energy where it is wanted
@@ -308,6 +317,10 @@ struct BoxLds {
     double w[kBox * kWPad];
     union {
         AtomLds rec[kBoxTile];
+        struct {
+            double after_rec[kBoxTile * sizeof(AtomLds) / sizeof(double)];
+            double node2[NG][kP2 * kP2 * kP2];
+        };
         struct {
             double t1[NG][4 * kP * kP];         // slab of 4 x: (x, node y, node z)
             double t2[NG][4 * kBox * kWPad];    // (x, y, node z)
@@ -335,11 +348,17 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
     const double cx = bx * kBox + half, cy = by * kBox + half, cz = bz * kBox + half;
     const double ccx = dcx * cx, ccy = dcy * cy, ccz = dcz * cz;
     const double hx = half * fabs(dcx), hy = half * fabs(dcy), hz = half * fabs(dcz);
-    const double dfar = fmax(kFarDist, kFarRatio * fmax(hx, fmax(hy, hz)));
-    auto is_far = [&](const AtomRec &a) {
+    const double hmax = fmax(hx, fmax(hy, hz));
+    // 0 near, 1 far, 2 very far
+    const bool two_sets = A.natoms > kBoxTile;
+    auto range = [&](const AtomRec &a) {
         const double rx = a.x - ccx, ry = a.y - ccy, rz = a.z - ccz;
         const double ex = fmax(fabs(rx) - hx, 0.0), ey = fmax(fabs(ry) - hy, 0.0), ez = fmax(fabs(rz) - hz, 0.0);
-        return ex * ex + ey * ey + ez * ez >= dfar * dfar && isfinite(rx) && isfinite(ry) && isfinite(rz);
+        const double d2 = (ex * ex + ey * ey + ez * ez);
+        // force terms 12 c12 r^-13 and 6 c6 r^-7
+        const bool far = d2 >= kFarRatio * kFarRatio * (hmax * hmax) && (!LJ || d2 * d2 * d2 * a.c6 >= 2.0 * kFarForces * a.c12) &&
+                         isfinite(rx) && isfinite(ry) && isfinite(rz);
+        return !far ? 0 : two_sets && d2 >= kVeryFarRatio * kVeryFarRatio * (hmax * hmax) ? 2 : 1;
     };
     for (int e = t; e < kBox * kP; e += kThreads) L.w[(e / kP) * kWPad + e % kP] = F.w[e];
 
@@ -365,12 +384,13 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
         for (int i0 = 0; i0 < A.natoms; i0 += kBoxTile) {
             const bool in = i0 + t < A.natoms;
             AtomRec a = {};
-            bool far = false;
+            int rg = -1;
             if (in) {
                 a = atoms[i0 + t];
-                far = is_far(a);
+                rg = range(a);
             }
-            const unsigned long long mf = __ballot(far), mn = __ballot(in && !far);
+            const bool far = rg == 1;
+            const unsigned long long mf = __ballot(far), mn = __ballot(rg == 0);
             if (lane == 0) {
                 L.count[0][wave] = __popcll(mf);
                 L.count[1][wave] = __popcll(mn);
@@ -391,7 +411,7 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
                 break;
             }
             if (far) L.rec[pf + __popcll(mf & below)] = atom_record(a, a.x - ccx, a.y - ccy, a.z - ccz);
-            else if (in) {
+            else if (rg == 0) {
                 const int p = pn + __popcll(mn & below);
                 if (p < kNearCap) L.list[p] = i0 + t;
             }
@@ -423,6 +443,81 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
         }
     }
     __syncthreads();
+    if (two_sets) {  // uniform
+        // ---- very far atoms at the second set of nodes
+        const int grp = t / (kP2 * kP2), c5 = t % (kP2 * kP2);
+        const bool on = grp < kGroups;
+        float nx[kP2], ny[kP2], nz[kP2];
+        double aL[kP2][4], aE[kP2][4];
+#pragma unroll
+        for (int k = 0; k < kP2; k++) {
+            nx[k] = (float)(F.x2[c5 / kP2] * half * dcx);
+            ny[k] = (float)(F.x2[c5 % kP2] * half * dcy);
+            nz[k] = (float)(F.x2[k] * half * dcz);
+#pragma unroll
+            for (int c = 0; c < 4; c++) { aL[k][c] = 0; aE[k][c] = 0; }
+        }
+        int any = 0;
+        for (int i0 = 0; i0 < A.natoms; i0 += kBoxTile) {
+            AtomRec a = {};
+            bool vf = false;
+            if (i0 + t < A.natoms) {
+                a = atoms[i0 + t];
+                vf = range(a) == 2;
+            }
+            const unsigned long long m = __ballot(vf);
+            if (lane == 0) L.count[0][wave] = __popcll(m);
+            __syncthreads();
+            int n = 0, p = 0;
+#pragma unroll
+            for (int q = 0; q < kThreads / 64; q++) {
+                if (q < wave) p += L.count[0][q];
+                n += L.count[0][q];
+            }
+            if (vf) L.rec[p + __popcll(m & ((1ull << lane) - 1))] = atom_record(a, a.x - ccx, a.y - ccy, a.z - ccz);
+            __syncthreads();
+            if (on)
+                sum_f32<LJ, NS, Z0, WE, QS, true, SEP, true, kP2>(A, L.rec, grp, kGroups, (n - grp + kGroups - 1) / kGroups, nx, ny,
+                                                                  nz, kP2, aL, aE);
+            any += n;
+            __syncthreads();
+        }
+        if (any > 0) {  // uniform
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                for (int r = 0; r < kGroups; r++) {  // the groups' sums, in order
+                    if (grp == r) {
+#pragma unroll
+                        for (int k = 0; k < kP2; k++)
+#pragma unroll
+                            for (int c = 0; c < NG; c++) {
+                                const double v = g == 0 ? aL[k][c] : aE[k][c];
+                                double &o = L.node2[c][c5 * kP2 + k];
+                                o = r == 0 ? v : o + v;
+                            }
+                    }
+                    __syncthreads();
+                }
+                for (int e = t; e < kP * kP * kP; e += kThreads) {
+                    double v[NG];
+#pragma unroll
+                    for (int c = 0; c < NG; c++) v[c] = 0;
+                    const double *wx = F.w2 + (e >> 6) * kP2, *wy = F.w2 + ((e >> 3) & 7) * kP2, *wz = F.w2 + (e & 7) * kP2;
+                    for (int i = 0; i < kP2 * kP2; i++) {
+                        const double wxy = wx[i / kP2] * wy[i % kP2];
+                        for (int k = 0; k < kP2; k++) {
+                            const double w = wxy * wz[k];
+#pragma unroll
+                            for (int c = 0; c < NG; c++) v[c] = __fma_rn(w, L.node2[c][i * kP2 + k], v[c]);
+                        }
+                    }
+#pragma unroll
+                    for (int c = 0; c < NG; c++) node[g][c][e] += v[c];
+                }
+                __syncthreads();
+            }
+        }
+    }
 
     // ---- the points, in slabs of 4 x: a wave holds 4x4 columns, a lane 4 z
     // points of one.  Near pairs are summed in coordinates relative to the
@@ -509,7 +604,7 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
             if (lane < nt) {
                 const AtomRec a = atoms[listed ? L.list[i0 + lane] : i0 + lane];
                 AtomLds r = atom_record(a, a.x - ox, a.y - oy, a.z - oz);
-                if (!listed && use_far && is_far(a)) {  // in the polynomial already: its terms here are zeros
+                if (!listed && use_far && range(a) > 0) {  // in the polynomial already: its terms here are zeros
                     r.hi.w = 0.f;
                     r.lj = make_float4(0.f, 0.f, 0.f, 0.f);
                 }
@@ -584,21 +679,27 @@ __global__ __launch_bounds__(kThreads, SEP ? 2 : 3) void ff_box_kernel(FFArgs A,
     box_f32<LJ, NS, Z0, WE, SEP>(A, F, atoms, out, (int)b);
 }
 
-FarTable make_far_table()
+// Chebyshev points of the first kind x[n] and the values w[m][n] of their
+// Lagrange polynomials at m points, none of them a node (barycentric form).
+void cheb(int n, double *x, int m, const double *at, double *w)
 {
     const double pi = 3.14159265358979323846;
-    FarTable F;
-    double bw[kP];  // barycentric weights of the Chebyshev points of the first kind
-    for (int k = 0; k < kP; k++) {
-        F.x[k] = std::cos((2 * k + 1) * pi / (2 * kP));
-        bw[k] = (k % 2 ? -1.0 : 1.0) * std::sin((2 * k + 1) * pi / (2 * kP));
-    }
-    for (int i = 0; i < kBox; i++) {  // no point coincides with a node
-        const double x = 2.0 * i / (kBox - 1) - 1.0;
+    for (int k = 0; k < n; k++) x[k] = std::cos((2 * k + 1) * pi / (2 * n));
+    for (int i = 0; i < m; i++) {
         double sum = 0;
-        for (int k = 0; k < kP; k++) sum += F.w[i * kP + k] = bw[k] / (x - F.x[k]);
-        for (int k = 0; k < kP; k++) F.w[i * kP + k] /= sum;
+        for (int k = 0; k < n; k++)
+            sum += w[i * n + k] = (k % 2 ? -1.0 : 1.0) * std::sin((2 * k + 1) * pi / (2 * n)) / (at[i] - x[k]);
+        for (int k = 0; k < n; k++) w[i * n + k] /= sum;
     }
+}
+
+FarTable make_far_table()
+{
+    FarTable F;
+    double pt[kBox];
+    for (int i = 0; i < kBox; i++) pt[i] = 2.0 * i / (kBox - 1) - 1.0;
+    cheb(kP, F.x, kBox, pt, F.w);
+    cheb(kP2, F.x2, kP, F.x, F.w2);
     return F;
 }
 

@@ -1,5 +1,6 @@
 """The FP32 grid of orthogonal cells: boxes of 16^3 points, atoms farther than
-8 half widths summed at 8^3 Chebyshev nodes (ff_grid_f32.hip box_f32), against
+8 half widths summed at 8^3 Chebyshev nodes, beyond 40 half widths at 5^3
+(ff_grid_f32.hip box_f32), against
 the FP64 oracle where that split can go wrong: too few far atoms for the
 polynomial (11) and just enough (12), one LDS tile of 256 atoms and one more,
 no far atom and no near atom at all, more near atoms than a box lists (512),
@@ -9,7 +10,8 @@ atom that is not finite.
 Bound at every point: |dF| <= 2e-6 S, S the sum over the atoms of the sizes of
 the terms that the kernel adds (repulsion and attraction, W / r0^3 and each
 w_s (1/r_s^3 - 1/r0^3) of the stencil): a term is rounded some 30 times at 6e-8
-each (1.8e-6), and the polynomial adds 8e-8 of the far atoms' force."""
+each (1.8e-6), and the polynomials add up to 5e-7 of the far atoms' force (their
+largest, Au at its limit; the rounding's 30 rarely all point one way)."""
 
 import numpy as np
 import pytest
@@ -103,6 +105,29 @@ def test_box_grid_vs_oracle(name, n, step, near, far, tip):
     _check(G, FE, _bound(n, L, xyz, qs, cLJs, tip))
     de = np.abs(G[..., 3] - FE[..., 3]) / np.maximum(np.abs(FE[..., 3]), 1e-3)
     assert de.max() < 1e-3
+
+
+@pytest.mark.parametrize("mode", ["dz2", "monopole", "separate"])
+@pytest.mark.parametrize("veryfar", [1, 11, 270])
+def test_second_set_of_nodes(mode, veryfar):
+    """More than one tile of atoms, some beyond 40 half widths (30 A): one, one more than the lane groups, a tile and more."""
+    n, L = (17, 20, 33), [1.7, 2.0, 3.3]
+    xyz = np.concatenate([_shell(veryfar // 2, L, 34.0, 80.0, 11).reshape(-1, 3), _shell(260, L, 3.0, 29.0, 12),
+                          _shell(veryfar - veryfar // 2, L, 34.0, 80.0, 13)])
+    qs, cLJs = _atoms(xyz, 8, uncharged=True)
+    if mode == "separate":
+        model = D.ff_model(0, with_lj=True, stencil=D.PROBE_STENCILS["s"], with_energy=True, coulomb_const=C.CoulombConst,
+                           probe_q=M.PROBE_Q, fmax=10.0, fp64_radius=0.0)
+        G = D.ff_build(n, np.diag(L), np.concatenate([xyz, qs[:, None]], 1), cLJs, model, f64=False).download()
+        FE = O.limit_vec_field(O.lj_ff(n, np.diag(L), xyz, cLJs), 10.0) + M.PROBE_Q * O.limit_vec_field(
+            O.coulomb_ff(n, np.diag(L), xyz, qs * C.CoulombConst), 10.0)
+        bound = _bound(n, L, xyz, qs, cLJs, ([abs(M.PROBE_Q)], [0.0]))
+    else:
+        tip = DZ2 if mode == "dz2" else MONOPOLE
+        G = _build(n, L, xyz, qs, cLJs, tip)
+        FE = O.ljc_qzs_ff(n, np.array([[0, 0, 0], *np.diag(L)]), np.concatenate([xyz, qs[:, None]], 1), cLJs, *tip)
+        bound = _bound(n, L, xyz, qs, cLJs, tip)
+    _check(G, FE, bound)
 
 
 def test_more_near_atoms_than_listed():
