@@ -75,6 +75,11 @@ __device__ __forceinline__ bf16x8 pack8(const unsigned short v[8])
     u.w = v[6] | ((unsigned)v[7] << 16);
     return __builtin_bit_cast(bf16x8, u);
 }
+// four bf16 in one store; p is 8-byte aligned
+__device__ __forceinline__ void store4(unsigned short *p, const unsigned short v[4])
+{
+    *(uint2 *)p = make_uint2(v[0] | ((unsigned)v[1] << 16), v[2] | ((unsigned)v[3] << 16));
+}
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -127,7 +132,7 @@ __global__ __launch_bounds__(64) void ws_fwd1_kernel(int S, const unsigned short
             for (int e = 0; e < 8; e++) {
                 const int off = tap_off(k0 + e);
                 v[e] = off >= 0 ? P[(long)s * kPatchStride + poff + off] : (unsigned short)0;
-                if (A1T) A1T[(long)(k0 + e) * (9L * S) + (long)s * 9 + p] = v[e];
+                if (A1T) A1T[(long)(k0 + e) * (9L * S) + (long)p * S + s] = v[e];
             }
             const bf16x8 a = pack8(v);
 #pragma unroll
@@ -139,17 +144,19 @@ __global__ __launch_bounds__(64) void ws_fwd1_kernel(int S, const unsigned short
         const int j = 16 * t + (l & 15);
         const float bj = net.theta[kOffB1 + j];
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 4; r++) {
+            const int s0 = 64 * tile + 16 * r + 4 * (l >> 4);
+            const int k2 = p * 32 + j;
+            unsigned short h[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int s = 64 * tile + 16 * r + 4 * (l >> 4) + i;
                 const float z = acc[r][t][i] + bj;
-                const unsigned short h = f2bf(silu(z));
-                const int k2 = p * 32 + j;
-                if (Z1) Z1[(long)s * kK2 + k2] = z;
-                H1[(long)s * kK2 + k2] = h;
-                if (H1T) H1T[(long)k2 * S + s] = h;
+                h[i] = f2bf(silu(z));
+                if (Z1) Z1[(long)(s0 + i) * kK2 + k2] = z;
+                H1[(long)(s0 + i) * kK2 + k2] = h[i];
             }
+            if (H1T) store4(H1T + (long)k2 * S + s0, h);  // 8 bytes: S and s0 are multiples of 4
+        }
     }
 }
 
@@ -193,15 +200,16 @@ __global__ __launch_bounds__(64) void ws_fwd2_kernel(int S, const unsigned short
 }
 
 // Layer 3, loss and the head of the backward pass; one thread per sample.
-// With grad, each block of 256 samples also leaves the sums of its samples'
+// With grad, each block of kHeadBlock samples also leaves the sums of its samples'
 // head gradient terms (dW3, db3, db2 and the loss, kHeadVals values) in
-// part[block]; ws_head_sum_kernel adds the blocks up in order (no atomics:
+// part[block]; ws_sum_kernel adds the blocks up in order (no atomics:
 // the same sums every run).  Samples s >= nvalid are padding: they produce
 // outputs but no gradient.
+constexpr int kHeadBlock = 64;  // 8192 samples: 128 blocks (256 a block left most CUs idle, 22 us)
 constexpr int kHeadVals = kN3 * kN2 + kN3 + kN2 + 1;
 constexpr int kHeadRow = kN3 + kN2 + kN2 + 2;  // dy, bf16(h), dz, loss term, pad: an odd stride of floats
 
-__global__ __launch_bounds__(256) void ws_head_kernel(int S, int nvalid, float inv_n, const float *__restrict__ Z2,
+__global__ __launch_bounds__(kHeadBlock) void ws_head_kernel(int S, int nvalid, float inv_n, const float *__restrict__ Z2,
                                                       const float *__restrict__ H2, Net net,
                                                       const float *__restrict__ T, float *__restrict__ out,
                                                       float *__restrict__ part, unsigned short *__restrict__ dZ2,
@@ -223,7 +231,7 @@ __global__ __launch_bounds__(256) void ws_head_kernel(int S, int nvalid, float i
         if (out && live) out[(long)s * kN3 + m] = a;
     }
     if (!part) return;  // uniform: forward only
-    __shared__ float sh[256][kHeadRow];
+    __shared__ float sh[kHeadBlock][kHeadRow];
     const int t = threadIdx.x;
     float dy[kN3], lsum = 0.f;
 #pragma unroll
@@ -251,34 +259,59 @@ __global__ __launch_bounds__(256) void ws_head_kernel(int S, int nvalid, float i
         }
     }
     __syncthreads();
-    // the block's sums: thread v < kHeadVals takes value v over the 256 samples
-    if (t < kHeadVals) {
+    // the block's sums: value v over its samples, in order
+    for (int v = t; v < kHeadVals; v += kHeadBlock) {
         float acc = 0.f;
-        if (t < kN3 * kN2) {  // dW3[m][j] = sum dy[m] bf16(h[j])
-            const int m = t / kN2, j = t % kN2;
-            for (int q = 0; q < 256; q++) acc = fmaf(sh[q][m], sh[q][kN3 + j], acc);
+        if (v < kN3 * kN2) {  // dW3[m][j] = sum dy[m] bf16(h[j])
+            const int m = v / kN2, j = v % kN2;
+            for (int q = 0; q < kHeadBlock; q++) acc = fmaf(sh[q][m], sh[q][kN3 + j], acc);
         } else {
             // db3 (dy), db2 (dz), the loss term
-            const int c = t < kN3 * kN2 + kN3 ? t - kN3 * kN2 : t < kN3 * kN2 + kN3 + kN2 ? kN3 + kN2 + (t - kN3 * kN2 - kN3)
+            const int c = v < kN3 * kN2 + kN3 ? v - kN3 * kN2 : v < kN3 * kN2 + kN3 + kN2 ? kN3 + kN2 + (v - kN3 * kN2 - kN3)
                                                                                             : kN3 + 2 * kN2;
-            for (int q = 0; q < 256; q++) acc += sh[q][c];
+            for (int q = 0; q < kHeadBlock; q++) acc += sh[q][c];
         }
-        part[(long)blockIdx.x * kHeadVals + t] = acc;
+        part[(long)blockIdx.x * kHeadVals + v] = acc;
     }
 }
 
-// The head's gradient and loss from the blocks' sums, added in block order.
-__global__ __launch_bounds__(256) void ws_head_sum_kernel(int nblocks, const float *__restrict__ part,
-                                                          float *__restrict__ grad, float *__restrict__ loss)
+// dW1 and the head's gradients and loss from the blocks' sums: a block takes
+// 64 values, its 16 groups of 64 threads every 16th partial sum each, and the
+// groups' sums are added in order (the same sums every run).  A chain of
+// dependent loads bounds it: one thread per value over 128 partial sums, in
+// two launches, took 40 us of a 147 us step.
+constexpr int kSumGroups = 16;
+__global__ __launch_bounds__(64 * kSumGroups) void ws_sum_kernel(int nb1, const float *__restrict__ part1, int nhb,
+                                                                 const float *__restrict__ part, float *__restrict__ grad,
+                                                                 float *__restrict__ loss)
 {
-    const int v = threadIdx.x;
-    if (v >= kHeadVals) return;
+    __shared__ float sh[kSumGroups][64];
+    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int n1 = kN1 * kK1;
+    int v = blockIdx.x * 64 + lane;
+    const bool w1 = v < n1;
     float acc = 0.f;
-    for (int b = 0; b < nblocks; b++) acc += part[(long)b * kHeadVals + v];
+    if (w1) {
+#pragma unroll 8
+        for (int b = g; b < nb1; b += kSumGroups) acc += part1[(long)b * n1 + v];
+    } else if (v < n1 + kHeadVals) {
+#pragma unroll 8
+        for (int b = g; b < nhb; b += kSumGroups) acc += part[(long)b * kHeadVals + (v - n1)];
+    }
+    sh[g][lane] = acc;
+    __syncthreads();
+    if (g != 0) return;
+    acc = 0.f;
+    for (int q = 0; q < kSumGroups; q++) acc += sh[q][lane];
+    if (w1) {
+        grad[kOffW1 + v] += acc;
+        return;
+    }
+    v -= n1;
     if (v < kN3 * kN2) grad[kOffW3 + v] += acc;
     else if (v < kN3 * kN2 + kN3) grad[kOffB3 + v - kN3 * kN2] += acc;
     else if (v < kHeadVals - 1) grad[kOffB2 + v - kN3 * kN2 - kN3] += acc;
-    else loss[0] += acc;
+    else if (v == kHeadVals - 1) loss[0] += acc;
 }
 
 // dW2[j][k2] += sum_s dZ2[s][j] H1[s][k2]: M = 32, N = 96 per block column,
@@ -319,7 +352,7 @@ __global__ __launch_bounds__(64) void ws_bwd2_kernel(int S, int ks, const unsign
 }
 
 // dA2 = dZ2 W2 (M = 64 samples, N = 288, K = 32), dZ1 = dA2 * silu'(Z1),
-// written transposed as dZ1T[c][s*9 + p]; db1.  Block (tile, y) takes the
+// written transposed as dZ1T[c][p*S + s]; db1.  Block (tile, y) takes the
 // 16-column slices 6y .. 6y+5 of the 18.
 __global__ __launch_bounds__(64) void ws_bwd1a_kernel(int S, const unsigned short *__restrict__ dZ2, Net net,
                                                        const float *__restrict__ Z1, unsigned short *__restrict__ dZ1T,
@@ -338,13 +371,15 @@ __global__ __launch_bounds__(64) void ws_bwd1a_kernel(int S, const unsigned shor
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             f32x4 d = mfma(a[r], b, f32x4{0.f, 0.f, 0.f, 0.f});
+            const int s0 = 64 * tile + 16 * r + 4 * (l >> 4);
+            unsigned short v[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int s = 64 * tile + 16 * r + 4 * (l >> 4) + i;
-                const float dz = d[i] * dsilu(Z1[(long)s * kK2 + k2]);
+                const float dz = d[i] * dsilu(Z1[(long)(s0 + i) * kK2 + k2]);
                 db[t & 1] += dz;
-                dZ1T[(long)c * (9L * S) + (long)s * 9 + p] = f2bf(dz);
+                v[i] = f2bf(dz);
             }
+            store4(dZ1T + (long)c * (9L * S) + (long)p * S + s0, v);
         }
     }
     // lanes l, l^16, l^32, l^48 hold the same channel
@@ -359,7 +394,7 @@ __global__ __launch_bounds__(64) void ws_bwd1a_kernel(int S, const unsigned shor
 
 // dW1[j][k] = sum_{(s,p)} dZ1[(s,p)][j] A1[(s,p)][k]: M = 32, N = 96, K = kr
 // rows of the (s,p) range per block, whose sums go to part[block][j][k]
-// (ws_w1_sum_kernel adds the blocks up in order).
+// (ws_sum_kernel adds the blocks up).
 __global__ __launch_bounds__(64) void ws_bwd1b_kernel(long K, int kr, const unsigned short *__restrict__ dZ1T,
                                                        const unsigned short *__restrict__ A1T, float *__restrict__ part)
 {
@@ -393,19 +428,6 @@ __global__ __launch_bounds__(64) void ws_bwd1b_kernel(long K, int kr, const unsi
             }
 }
 
-// dW1 from ws_bwd1b_kernel's block sums, added in block order.
-__global__ __launch_bounds__(256) void ws_w1_sum_kernel(int nblocks, const float *__restrict__ part,
-                                                        float *__restrict__ grad)
-{
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= kN1 * kK1) return;
-    float acc = 0.f;
-    for (int b = 0; b < nblocks; b++) acc += part[(long)b * (kN1 * kK1) + v];
-    grad[kOffW1 + v] += acc;
-}
-
-// Adam on the FP32 master parameters; refreshes the bf16 copies and clears
-// the gradient.  step >= 1.
 __global__ __launch_bounds__(256) void ws_adam_kernel(float *__restrict__ theta, float *__restrict__ grad,
                                                       float *__restrict__ m1, float *__restrict__ m2, float lr,
                                                       float beta1, float beta2, float eps, float c1, float c2,
@@ -991,7 +1013,7 @@ int ws_alloc(WsModel &m, int cap)
     PP_TRY_HIP(hipMalloc((void **)&m.dZ1T, c * 9 * kN1 * 2));
     PP_TRY_HIP(hipMalloc((void **)&m.Ppad, c * kPatchStride * 2));
     PP_TRY_HIP(hipMalloc((void **)&m.Tpad, c * kN3 * 4));
-    PP_TRY_HIP(hipMalloc((void **)&m.part, ((c + 255) / 256) * kHeadVals * 4));
+    PP_TRY_HIP(hipMalloc((void **)&m.part, ((c + kHeadBlock - 1) / kHeadBlock) * kHeadVals * 4));
     PP_TRY_HIP(hipMalloc((void **)&m.part1, (9 * c / kW1Rows) * (kN1 * kK1) * 4));
     return 0;
 }
@@ -1023,11 +1045,10 @@ int ws_pass(WsModel &m, int S, int nvalid, const unsigned short *P, const float 
                        train ? m.H1T : nullptr, train ? m.A1T : nullptr);
     hipLaunchKernelGGL(ws_fwd2_kernel, dim3(S / 64), dim3(64), 0, st, S, m.H1, net, m.Z2, m.H2);
     const float inv_n = nvalid > 0 ? 1.f / (3.f * (float)nvalid) : 0.f;
-    const int nhb = (S + 255) / 256;
-    hipLaunchKernelGGL(ws_head_kernel, dim3(nhb), dim3(256), 0, st, S, nvalid, inv_n, m.Z2, m.H2, net, T, out,
+    const int nhb = (S + kHeadBlock - 1) / kHeadBlock;
+    hipLaunchKernelGGL(ws_head_kernel, dim3(nhb), dim3(kHeadBlock), 0, st, S, nvalid, inv_n, m.Z2, m.H2, net, T, out,
                        train ? m.part : nullptr, m.dZ2, m.dZ2T);
     if (!train) return 0;
-    hipLaunchKernelGGL(ws_head_sum_kernel, dim3(1), dim3(256), 0, st, nhb, m.part, m.grad, m.loss);
     // dW2: K = S split into chunks of up to 512 samples
     int ks = 512;
     while (S % ks) ks >>= 1;
@@ -1038,7 +1059,8 @@ int ws_pass(WsModel &m, int S, int nvalid, const unsigned short *P, const float 
     const long K = 9L * S;
     const int nb1 = (int)(K / kW1Rows);
     hipLaunchKernelGGL(ws_bwd1b_kernel, dim3((unsigned)nb1), dim3(64), 0, st, K, kW1Rows, m.dZ1T, m.A1T, m.part1);
-    hipLaunchKernelGGL(ws_w1_sum_kernel, dim3((kN1 * kK1 + 255) / 256), dim3(256), 0, st, nb1, m.part1, m.grad);
+    hipLaunchKernelGGL(ws_sum_kernel, dim3((kN1 * kK1 + kHeadVals + 63) / 64), dim3(64 * kSumGroups), 0, st, nb1, m.part1, nhb,
+                       m.part, m.grad, m.loss);
     return 0;
 }
 
