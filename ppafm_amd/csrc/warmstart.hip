@@ -132,7 +132,7 @@ __global__ __launch_bounds__(64) void ws_fwd1_kernel(int S, const unsigned short
             for (int e = 0; e < 8; e++) {
                 const int off = tap_off(k0 + e);
                 v[e] = off >= 0 ? P[(long)s * kPatchStride + poff + off] : (unsigned short)0;
-                if (A1T) A1T[(long)(k0 + e) * (9L * S) + (long)p * S + s] = v[e];
+                if (A1T) A1T[(long)(k0 + e) * (9L * S) + (long)s * 9 + p] = v[e];
             }
             const bf16x8 a = pack8(v);
 #pragma unroll
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(64) void ws_bwd2_kernel(int S, int ks, const unsign
 }
 
 // dA2 = dZ2 W2 (M = 64 samples, N = 288, K = 32), dZ1 = dA2 * silu'(Z1),
-// written transposed as dZ1T[c][p*S + s]; db1.  Block (tile, y) takes the
+// written transposed as dZ1T[c][s*9 + p]; db1.  Block (tile, y) takes the
 // 16-column slices 6y .. 6y+5 of the 18.
 __global__ __launch_bounds__(64) void ws_bwd1a_kernel(int S, const unsigned short *__restrict__ dZ2, Net net,
                                                        const float *__restrict__ Z1, unsigned short *__restrict__ dZ1T,
@@ -372,14 +372,13 @@ __global__ __launch_bounds__(64) void ws_bwd1a_kernel(int S, const unsigned shor
         for (int r = 0; r < 4; r++) {
             f32x4 d = mfma(a[r], b, f32x4{0.f, 0.f, 0.f, 0.f});
             const int s0 = 64 * tile + 16 * r + 4 * (l >> 4);
-            unsigned short v[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const float dz = d[i] * dsilu(Z1[(long)(s0 + i) * kK2 + k2]);
                 db[t & 1] += dz;
-                v[i] = f2bf(dz);
+                // (position fastest; samples fastest and 8-byte stores took 26 us for 21 here)
+                dZ1T[(long)c * (9L * S) + (long)(s0 + i) * 9 + p] = f2bf(dz);
             }
-            store4(dZ1T + (long)c * (9L * S) + (long)p * S + s0, v);
         }
     }
     // lanes l, l^16, l^32, l^48 hold the same channel
