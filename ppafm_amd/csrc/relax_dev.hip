@@ -351,7 +351,7 @@ constexpr int stage_batch()
 }
 
 // A wave relaxes a tile of A.tile_x x A.tile_y columns (64 or fewer, its
-// remaining lanes idle).  Block b runs its waves' consecutive tiles of part
+// remaining lanes idle), or that many consecutive ones (A.tiles_y 0).  Block b runs its waves' consecutive tiles of part
 // b % 8 (one contiguous part of the tiles per XCD).
 // FRAC 0 in tiles of a few columns, where lanes seldom wait together.
 template <typename T4, int MODE, bool ORTHO, int WPB, int FRAC>
@@ -366,8 +366,16 @@ __global__ __launch_bounds__(64 * WPB) void relax_dev_kernel(DevArgs A, const T4
     const int tile = ((b % 8) * per_xcd + b / 8) * WPB + wave;
     if (tile >= A.ntiles) return;
     Stage<kStageSingle> G = make_stage<kStageSingle>(single_lds, cols * WPB, wave * cols + min(lane, cols - 1));
-    const int ti = tile / A.tiles_y, tj = tile % A.tiles_y;
-    const int i = ti * A.tile_x + lane / A.tile_y, j = tj * A.tile_y + lane % A.tile_y;
+    int i, j;
+    if (A.tiles_y > 0) {
+        const int ti = tile / A.tiles_y, tj = tile % A.tiles_y;
+        i = ti * A.tile_x + lane / A.tile_y;
+        j = tj * A.tile_y + lane % A.tile_y;
+    } else {  // consecutive columns: every wave but the last is full
+        const int c = tile * cols + lane;
+        i = c / A.ny;
+        j = c - i * A.ny;
+    }
     unsigned long long nevals = 0, npos = 0;
     unsigned turns = 0;
     relax_column<T4, MODE, kStageSingle, ORTHO, FRAC>(A, grid, i, j, lane < cols && i < A.nx && j < A.ny, G, nevals, npos, turns);
@@ -580,21 +588,26 @@ static int simd_count()
 
 // Single-scan launch.  A column's steps are a serial chain, so a scan takes
 // as long as its slowest wave, and a wave is faster the fewer columns it holds
-// (its lanes reach new cells and step ends at different passes).  Tiles are
-// therefore as small as the SIMDs allow, one wave each: the smallest power of
-// two of columns that leaves no more tiles than SIMDs, 4 at least (2 and 1 run
-// the same or slower) and 64 at most.  Relaxation alone, 64 columns a wave
-// against this: 24x24x20 scan (4 columns) 1.75 -> 1.54 ms, 128x128x40 (16)
-// 2.89 -> 2.73, 128x128x30 OpenCL semantics (16) 0.86 -> 0.70; half as many
-// columns again, two waves on a SIMD, is slower: 128x128x40 (8) 4.98,
-// 256x256x60 (32 against 64) 8.15 against 6.17.
-// With one-wave workgroups the dispatcher has been seen to place two waves of
-// such a launch on one SIMD while another SIMD of the CU idles, depending on
-// what ran before it (256x256x60: 8.9-9.3 ms against 7.1-7.4; 128x128x40 3.65
-// against 2.65).  A scan with more than 3 tiles per CU and at most one per
-// SIMD uses four-wave workgroups, one per CU with its waves on the CU's four
-// SIMDs.  Others keep one-wave workgroups spread over the CUs (four-wave
-// workgroups there leave CUs idle), and so do scans beyond one tile per SIMD.
+// (its lanes reach new cells and step ends at different passes) as long as it
+// has a SIMD to itself.  Measured, whole call of a 30-step scan of 60 atoms on
+// 160x160x130 points, columns a wave / waves a workgroup (64 / 1 before: 3.0
+// to 3.1 ms at each size):
+//   24x24    4/1 1.78  8/1 1.90  16/1 2.14  4/4 3.31
+//   33x47    8/1 1.91  16/1 2.19  4/1 (408 waves) 2.26  4/4 3.45
+//   48x48    16/1 2.15  16/4 2.20  8/1 (288) 2.34  8/4 3.46  4/1 (576) 2.83
+//   64x64    16/4 2.03  16/1 2.27  8/1 2.54  8/4 3.78  4/1 3.75
+//   128x128  16/4 1.95  32/4 2.28  64/1 2.33  16/1 2.74
+//   181x181  64/4 2.42  32/4 (1,058 waves) 3.62
+// So: 4, then 8 columns while one-wave workgroups are at most one a CU, then
+// 16, 32 and 64 while there are no more waves than SIMDs, four a workgroup and
+// a CU as soon as they are more than the CUs (one-wave workgroups may put two
+// waves on one SIMD of a CU: 16/1 above).  Waves with 8 active lanes or fewer
+// run at half the speed where a CU holds several (4/4, 8/4; 4x4 tiles of a
+// 70x70 scan, whose edge tiles have 8 columns, 3.1 ms): below 32 columns a wave
+// takes consecutive columns, so that none but the last is short (70x70 2.0,
+// 65x65 3.2 -> 2.0).  Scans beyond one wave of 64 columns per SIMD keep
+// one-wave workgroups.  Waves of 32 and 64 columns let lanes wait (serve): at
+// 128x128 64 columns 2.33 ms against 2.82, but 16 columns 2.26 against 1.95.
 template <typename T4, int MODE, bool ORTHO, int WPB, int FRAC>
 static void launch_single_w(const DevArgs &A, const void *grid, hipStream_t st)
 {
@@ -610,25 +623,23 @@ static void launch_single(const DevArgs &A0, const void *grid, hipStream_t st)
     const int simds = simd_count();
     const int cus = simds / 4;
     DevArgs A = A0;
-    static const int tiles[][2] = {{2, 2}, {4, 2}, {4, 4}, {8, 4}, {8, 8}};
+    static const int tiles[][2] = {{1, 4}, {1, 8}, {1, 16}, {8, 4}, {8, 8}};
     for (const auto &t : tiles) {
+        const int cols = t[0] * t[1];
         A.tile_x = t[0];
         A.tile_y = t[1];
-        A.tiles_y = (A.ny + t[1] - 1) / t[1];
-        const long n = ((A.nx + t[0] - 1L) / t[0]) * A.tiles_y;
-        if (n <= simds || t[0] * t[1] == 64) {
+        A.tiles_y = cols < 32 ? 0 : (A.ny + t[1] - 1) / t[1];
+        const long n = cols < 32 ? ((long)A.nx * A.ny + cols - 1) / cols : ((A.nx + t[0] - 1L) / t[0]) * A.tiles_y;
+        if (n <= (cols < 16 ? cus : simds) || cols == 64) {
             A.ntiles = (int)n;
             break;
         }
     }
-    const bool wide = A.tile_x * A.tile_y >= 16;
-    if (wide && cus > 0 && A.ntiles > 3L * cus && A.ntiles <= simds) {
-        launch_single_w<T4, MODE, ORTHO, 4, kServe[MODE]>(A, grid, st);
-    } else if (wide) {
-        launch_single_w<T4, MODE, ORTHO, 1, kServe[MODE]>(A, grid, st);
-    } else {
-        launch_single_w<T4, MODE, ORTHO, 1, 0>(A, grid, st);
-    }
+    const bool wide = A.tile_x * A.tile_y >= 32, four = cus > 0 && A.ntiles > cus && A.ntiles <= simds;
+    if (wide && four) launch_single_w<T4, MODE, ORTHO, 4, kServe[MODE]>(A, grid, st);
+    else if (wide) launch_single_w<T4, MODE, ORTHO, 1, kServe[MODE]>(A, grid, st);
+    else if (four) launch_single_w<T4, MODE, ORTHO, 4, 0>(A, grid, st);
+    else launch_single_w<T4, MODE, ORTHO, 1, 0>(A, grid, st);
 }
 
 int launch_relax_fast(const RelaxLaunch &L, const void *grid, bool f64, hipStream_t st)

@@ -1,8 +1,8 @@
 """Tile sizes of the single-scan relaxation (launch_single, relax_dev.hip): a
 scan of any size, in tiles of 4 to 64 columns with and without waiting lanes,
 gives the bits of the batch kernel, whose tiles have 64 columns.  Sizes: one
-column, ragged ones, 1,024 SIMDs' worth of tiles of 4, 16 and 32 columns
-exactly and one row more."""
+column, ragged ones, and on 256 CUs and 1,024 SIMDs the last of 4, 8, 16 and 32
+columns a wave (32x32, 64x32, 128x128, 256x128) and one row more."""
 
 import numpy as np
 import pytest
@@ -19,7 +19,7 @@ LVEC = np.array([[-3.2, -3.2, -3.0], [6.4, 0, 0], [0, 6.4, 0], [0, 0, 12.0]])
 N = (64, 64, 120)
 
 
-@pytest.mark.parametrize("nx,ny", [(1, 1), (3, 5), (24, 24), (64, 64), (65, 64), (91, 90), (128, 128), (129, 128), (181, 181), (256, 128), (256, 129)])
+@pytest.mark.parametrize("nx,ny", [(1, 1), (3, 5), (32, 32), (33, 32), (64, 32), (65, 32), (64, 64), (70, 70), (91, 90), (128, 128), (129, 128), (181, 181), (256, 128), (256, 129)])
 def test_single_scan_equals_batch(nx, ny):
     print(f"case: {nx} x {ny} columns", flush=True)
     scan = dict(scan_n=(nx, ny), scan_x=(-2.5, 2.5), scan_y=(-2.5, 2.5), z_top=6.2, nz=3, dz=0.1)
