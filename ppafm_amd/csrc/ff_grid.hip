@@ -508,9 +508,9 @@ static bool model_args(const ppafm_ff_model &m, FFArgs &A)
     A.fmax = m.fmax;
     // FP64 radius: at least 0.2 A beyond the farthest stencil offset, so no
     // FP32 pair (LJ or shifted Coulomb point) comes closer than 0.2 A
-    double maxdz = 0;
-    for (int s = 0; s < ns; s++) maxdz = fmax(maxdz, fabs((double)A.sdz[s]));
-    const double rmin = kMinFp64Radius + maxdz;
+    A.maxdz = 0.f;
+    for (int s = 0; s < ns; s++) A.maxdz = fmaxf(A.maxdz, fabsf(A.sdz[s]));
+    const double rmin = kMinFp64Radius + (double)A.maxdz;
     const double rn = m.fp64_radius > rmin ? m.fp64_radius : rmin;
     A.near2 = (float)(rn * rn);
     return zi >= 0;

@@ -270,8 +270,9 @@ __device__ __forceinline__ void brick_f32(const FFArgs &A, const AtomRec *__rest
 }
 
 // Orthogonal cells: a block computes a box of 16^3 points.  The field of an
-// atom farther from the box than kFarRatio half widths, and so far that its
-// repulsion is below 1/24 of its attraction, is smooth over it: such far atoms
+// atom farther from the box than kFarRatio half widths (with the Coulomb
+// stencil's points, which lie up to maxdz above and below it), and so far that
+// its repulsion is below 1/24 of its attraction, is smooth over it: such far atoms
 // are summed at the box's kP^3 Chebyshev nodes only, and the sums are carried
 // to the 4096 points by the nodes' tensor-product polynomial in FP64; atoms
 // nearer are summed at every point.  A far pair costs 1/8 of a near one.  With
@@ -353,10 +354,13 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
     const bool two_sets = A.natoms > kBoxTile;
     auto range = [&](const AtomRec &a) {
         const double rx = a.x - ccx, ry = a.y - ccy, rz = a.z - ccz;
-        const double ex = fmax(fabs(rx) - hx, 0.0), ey = fmax(fabs(ry) - hy, 0.0), ez = fmax(fabs(rz) - hz, 0.0);
+        // the stencil's Coulomb points act as charges up to maxdz above and
+        // below the atom: the distance is that of the nearest of them
+        const double ex = fmax(fabs(rx) - hx, 0.0), ey = fmax(fabs(ry) - hy, 0.0), ez = fmax(fabs(rz) - (hz + A.maxdz), 0.0);
         const double d2 = (ex * ex + ey * ey + ez * ez);
         // force terms 12 c12 r^-13 and 6 c6 r^-7
-        const bool far = d2 >= kFarRatio * kFarRatio * (hmax * hmax) && (!LJ || d2 * d2 * d2 * a.c6 >= 2.0 * kFarForces * a.c12) &&
+        const bool far = d2 >= kFarRatio * kFarRatio * (hmax * hmax) &&
+                         (!LJ || d2 * d2 * d2 * a.c6 >= 2.0 * kFarForces * fabs(a.c12)) &&
                          isfinite(rx) && isfinite(ry) && isfinite(rz);
         return !far ? 0 : two_sets && d2 >= kVeryFarRatio * kVeryFarRatio * (hmax * hmax) ? 2 : 1;
     };

@@ -184,3 +184,62 @@ def test_batch_of_many_atoms_equals_single_grids():
         G = D.ff_build(n, lvec[1:], np.concatenate([xyz - lvec[0], qs[:, None]], 1), cLJs, b.model, f64=False).download()
         assert np.array_equal(b.grid(k), G), k
     b.close()
+
+
+def _offset_bound(n, L, xyz, qs, cLJs, tip, ke=14.399644):
+    """_bound, and the rounding of a stencil point's distance: its z is the
+    sum of two numbers of up to |dz| and |z|, each rounded at 6e-8, and the
+    charge's field changes by at most 2 / rs^3 per A."""
+    ax = [np.arange(m) * (l / m) for m, l in zip(n, L)]
+    S = _bound(n, L, xyz, qs, cLJs, tip, ke)
+    for p, q in zip(xyz, qs):
+        d = [a - v for a, v in zip(ax, p)]
+        rxy2 = (d[0] ** 2)[:, None, None] + (d[1] ** 2)[None, :, None]
+        for w, z in zip(*tip):
+            rs = np.sqrt(rxy2 + ((d[2] + z) ** 2)[None, None, :])
+            S = S + abs(q * w) * ke * 2 / rs**3 * (6e-8 * (2 * np.abs(d[2]) + abs(z)))[None, None, :]
+    return S
+
+
+@pytest.mark.parametrize("lj", ["without LJ", "zero coefficients", "LJ"])
+@pytest.mark.parametrize("step", [0.02, 0.05, 0.1])
+@pytest.mark.parametrize("offset", [1.0, -2.5, 3.0, -6.0, 8.0])
+def test_stencil_points_reach_the_box(offset, step, lj):
+    """Atoms more than 8 half widths from the box whose stencil points (the
+    tip's z offset) lie beside the box or inside it, and as many whose points
+    stay far away: the first must not be summed at the nodes."""
+    n, L = (16, 16, 16), [16 * step] * 3
+    rng = np.random.default_rng(7)
+    near, lo = 7.5 * step, max(8.2 * 7.5 * step, 2.0 if lj == "LJ" else 0.0)  # half width, distance from the box
+    xyz = []
+    while len(xyz) < 24:
+        p = rng.uniform(-2 * near, L[0] + 2 * near, 3)
+        p[2] += offset * rng.uniform(0.8, 1.0)  # its charge at dz + offset: beside the box
+        if np.linalg.norm(np.maximum(np.maximum(-p, p - L[0]), 0)) >= lo:
+            xyz.append(p)
+        elif abs(offset) + 2 * near < lo:  # no such atom at this offset: as close as they come
+            xyz.append(p + np.array([0, 0, np.sign(offset) * lo]))
+    xyz = np.concatenate([np.array(xyz), _shell(24, L, max(lo, 6.1), 20.0, 3)])
+    qs, cLJs = _atoms(xyz, 4)
+    if lj != "LJ":
+        cLJs = np.zeros_like(cLJs)
+    tip = (np.array([-0.1, 0.05, 0, 0]), np.array([0.0, offset, 0, 0]))
+    model = D.ff_model(1, with_lj=lj != "without LJ", stencil=list(zip(*tip)), with_energy=True, fmax=None)
+    G = D.ff_build(n, np.diag(L), np.concatenate([xyz, qs[:, None]], 1), cLJs, model, f64=False).download()
+    FE = O.ljc_qzs_ff(n, np.array([[0, 0, 0], *np.diag(L)]), np.concatenate([xyz, qs[:, None]], 1), cLJs, *tip)
+    _check(G, FE, _offset_bound(n, L, xyz, qs, cLJs, tip))
+
+
+@pytest.mark.parametrize("offset", [6.0, -31.0])
+def test_stencil_points_of_very_far_atoms(offset):
+    """More than 256 atoms just beyond 40 half widths (30 A) above and below
+    the box, whose stencil points lie within them, at 31 A inside the box."""
+    n, L = (17, 16, 16), [1.7, 1.6, 1.6]
+    rng = np.random.default_rng(1)
+    xyz = np.concatenate([rng.uniform([-3, -3, 0], [4.7, 4.6, 1], (300, 3)), _shell(20, L, 3.0, 12.0, 2)])
+    xyz[:300, 2] = np.where(np.arange(300) % 2, L[2] + rng.uniform(30.1, 34, 300), -rng.uniform(30.1, 34, 300))
+    qs, cLJs = _atoms(xyz, 6)
+    tip = (np.array([-0.1, 0.05, 0, 0]), np.array([0.0, offset, 0, 0]))
+    G = _build(n, L, xyz, qs, cLJs, tip)
+    FE = O.ljc_qzs_ff(n, np.array([[0, 0, 0], *np.diag(L)]), np.concatenate([xyz, qs[:, None]], 1), cLJs, *tip)
+    _check(G, FE, _offset_bound(n, L, xyz, qs, cLJs, tip))
