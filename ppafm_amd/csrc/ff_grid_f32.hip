@@ -138,13 +138,13 @@ __device__ __forceinline__ void atom_f32(const FFArgs &A, const AtomLds &a, cons
 }
 
 // Sums over the atoms lds[first], lds[first + step], ... (n of them) at the
-// lane's points: FP32 partial sums of kFold atoms folded into FP64.
-template <bool LJ, int NS, bool Z0, bool WE, bool QS, bool ORTHO, bool SEP, bool ALL, int K = kK>
+// lane's points: FP32 partial sums of FOLD atoms folded into FP64.
+template <bool LJ, int NS, bool Z0, bool WE, bool QS, bool ORTHO, bool SEP, bool ALL, int K = kK, int FOLD = kFold>
 __device__ __forceinline__ void sum_f32(const FFArgs &A, const AtomLds *lds, int first, int step, int n, const float *px,
                                         const float *py, const float *pz, int nk, double aL[K][4], double aE[K][4])
 {
-    for (int j0 = 0; j0 < n; j0 += kFold) {
-        const int j1 = min(n, j0 + kFold);
+    for (int j0 = 0; j0 < n; j0 += FOLD) {
+        const int j1 = min(n, j0 + FOLD);
         float sL[K][4], sE[K][4];
 #pragma unroll
         for (int k = 0; k < K; k++)
@@ -280,16 +280,24 @@ __device__ __forceinline__ void brick_f32(const FFArgs &A, const AtomRec *__rest
 // summed at kP2^3 nodes (1/33), whose polynomial is added to the values at the
 // kP^3 nodes.  VALU bound as before, in the near pairs for a molecule, in the
 // nodes for a slab.
-// Interpolation error, against the far atom's own force on 0.1 A steps: order
-// 8 at ratio 8 (6 A) 8e-8 for C, H, N, O and 5e-7 for Au at its 6.9 A; order 5
-// at ratio 40 (30 A) 3e-7 of the Lennard-Jones force, 5e-9 of the Coulomb
-// force.  The FP32 pair sums' own rounding is 4e-7 of the total at the median
-// point of a slab's grid and 2e-6 at the 99th percentile, before and after.
-// Order 7, or ratio 6.7, loses a digit at 6 A; order 4 at 30 A two.
+// Interpolation error at 0.1 A steps, against the far atom's own force at the
+// point, largest over a box that faces the atom (an atom off its edges or
+// corners: a tenth), in FP64: order 8 at ratio 8 (6 A) 5.9e-7 for H, 4.1e-7 O,
+// 2.7e-7 N, 1.3e-7 C (6.1 A), 3e-8 Au (6.9 A), 4e-9 of the Coulomb force; its
+// root mean square over the box is a third of that.  Order 5 at ratio 40 (30 A):
+// 3.5e-7 of the Lennard-Jones force, 5e-9 of the Coulomb force.  An FP32 pair is
+// rounded by as much, which is why the grid's error as a whole may not grow:
+// the nodes are stretched to the box's ends, where the polynomial would
+// otherwise scale a node's rounding by up to 1.4 an axis (now at most 1.02), and
+// their FP32 sums are 8 atoms long, not 32.  Over 17 grids (slabs and molecules,
+// both tips) the error against FP64 is 0.90 (median) and 0.95 (99th percentile)
+// of the sum over every pair, 0.92 and 0.90 for the energy; without these two
+// changes it was 1.02 and 1.08, 1.18 and 1.17.  Node coordinates are FP32 while
+// the weights assume exact nodes: 3e-8 A at 0.75 A, 4e-8 of the force at 6 A.
 // Measured (grid kernel, before: every atom at every point): 60 atoms, dz2
 // tip, 256x256x192 points 1277 -> 373 us; 16 such grids of 8-120 atoms
 // 23.5 -> 6.6 ms; 17,928 atoms, 400x400x300 points 321 -> 43 ms with one set of
-// nodes, 14.7 ms with two.
+// nodes, 15.3 ms with two.
 constexpr int kBox = 16;
 constexpr int kP = 8;
 constexpr double kFarRatio = 8.0;
@@ -300,12 +308,14 @@ constexpr int kGroups = 10;  // lane groups of kP2^2 that share the atoms, kP2 n
 // Far atoms a box needs before the polynomial (56 FP64 FMAs per point) costs
 // less than their pair sums; below it every atom of the box counts as near.
 constexpr int kFarMin = 12;
+constexpr int kNodeFold = 8;  // FP32 partial-sum length at the nodes
 constexpr int kBoxTile = kThreads;  // atoms per LDS tile, one per thread
 constexpr int kNearCap = 512;       // near atoms listed; beyond, every atom is staged for each slab
 constexpr int kWPad = kP + 1;       // row stride against LDS bank conflicts
 
-// Chebyshev nodes on [-1, 1] and the values of their Lagrange polynomials at
-// the box's equidistant points (the ends at -1 and 1).
+// Chebyshev nodes, stretched so that the first and last are -1 and 1, and the
+// values of their Lagrange polynomials at the box's equidistant points (the
+// ends at -1 and 1).
 struct FarTable {
     double x[kP];
     double w[kBox * kP];
@@ -421,7 +431,8 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
             }
             __syncthreads();
             const int first = t >> 7;
-            sum_f32<LJ, NS, Z0, WE, QS, true, SEP, true>(A, L.rec, first, 2, (nf - first + 1) / 2, nx, ny, nz, kK, aL, aE);
+            sum_f32<LJ, NS, Z0, WE, QS, true, SEP, true, kK, kNodeFold>(A, L.rec, first, 2, (nf - first + 1) / 2, nx, ny, nz, kK,
+                                                                        aL, aE);
             __syncthreads();
         }
         if (use_far) {
@@ -481,8 +492,9 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
             if (vf) L.rec[p + __popcll(m & ((1ull << lane) - 1))] = atom_record(a, a.x - ccx, a.y - ccy, a.z - ccz);
             __syncthreads();
             if (on)
-                sum_f32<LJ, NS, Z0, WE, QS, true, SEP, true, kP2>(A, L.rec, grp, kGroups, (n - grp + kGroups - 1) / kGroups, nx, ny,
-                                                                  nz, kP2, aL, aE);
+                sum_f32<LJ, NS, Z0, WE, QS, true, SEP, true, kP2, kNodeFold>(A, L.rec, grp, kGroups,
+                                                                             (n - grp + kGroups - 1) / kGroups, nx, ny, nz, kP2,
+                                                                             aL, aE);
             any += n;
             __syncthreads();
         }
@@ -683,13 +695,21 @@ __global__ __launch_bounds__(kThreads, SEP ? 2 : 3) void ff_box_kernel(FFArgs A,
     box_f32<LJ, NS, Z0, WE, SEP>(A, F, atoms, out, (int)b);
 }
 
-// Chebyshev points of the first kind x[n] and the values w[m][n] of their
-// Lagrange polynomials at m points, none of them a node (barycentric form).
+// Chebyshev points of the first kind, divided by the largest (which leaves
+// their barycentric weights), x[n], and the values w[m][n] of their Lagrange
+// polynomials at m points (barycentric form; unit weights at a node).
 void cheb(int n, double *x, int m, const double *at, double *w)
 {
     const double pi = 3.14159265358979323846;
-    for (int k = 0; k < n; k++) x[k] = std::cos((2 * k + 1) * pi / (2 * n));
+    for (int k = 0; k < n; k++) x[k] = std::cos((2 * k + 1) * pi / (2 * n)) / std::cos(pi / (2 * n));
     for (int i = 0; i < m; i++) {
+        int node = -1;
+        for (int k = 0; k < n; k++)
+            if (std::fabs(at[i] - x[k]) < 1e-12) node = k;
+        if (node >= 0) {
+            for (int k = 0; k < n; k++) w[i * n + k] = k == node;
+            continue;
+        }
         double sum = 0;
         for (int k = 0; k < n; k++)
             sum += w[i * n + k] = (k % 2 ? -1.0 : 1.0) * std::sin((2 * k + 1) * pi / (2 * n)) / (at[i] - x[k]);

@@ -10,8 +10,10 @@ atom that is not finite.
 Bound at every point: |dF| <= 2e-6 S, S the sum over the atoms of the sizes of
 the terms that the kernel adds (repulsion and attraction, W / r0^3 and each
 w_s (1/r_s^3 - 1/r0^3) of the stencil): a term is rounded some 30 times at 6e-8
-each (1.8e-6), and the polynomials add up to 5e-7 of the far atoms' force (their
-largest, Au at its limit; the rounding's 30 rarely all point one way)."""
+each (1.8e-6; the 30 rarely all point one way), and the polynomials add up to
+6e-7 of a far atom's force (H, 6 A from a side of its box).  For the dz2 tip S is
+the sizes of stencil terms that cancel, so the error as a whole is compared with
+that of the sum over every pair too."""
 
 import numpy as np
 import pytest
@@ -243,3 +245,46 @@ def test_stencil_points_of_very_far_atoms(offset):
     G = _build(n, L, xyz, qs, cLJs, tip)
     FE = O.ljc_qzs_ff(n, np.array([[0, 0, 0], *np.diag(L)]), np.concatenate([xyz, qs[:, None]], 1), cLJs, *tip)
     _check(G, FE, _offset_bound(n, L, xyz, qs, cLJs, tip))
+
+
+def _slab(z, half, count):
+    """Six layers of a square net of Au atoms below z, displaced at random by
+    0.05 A (atoms of one height would all round alike), the count nearest to the axis."""
+    rng = np.random.default_rng(1)
+    ax = np.arange(-half, half + 2.9, 2.9)
+    p = np.stack(np.meshgrid(ax, ax, z - 2.35 * np.arange(6), indexing="ij"), -1).reshape(-1, 3)
+    return (p + rng.normal(0, 0.05, p.shape))[np.argsort((p[:, :2] ** 2).sum(1), kind="stable")[:count]] + [0.8, 0.8, 0]
+
+
+SYSTEMS = ["molecule", "ring", "slab", "far slab"]
+
+
+@pytest.mark.parametrize("tip", [DZ2, MONOPOLE], ids=["dz2", "monopole"])
+@pytest.mark.parametrize("system", SYSTEMS)
+def test_error_no_larger_than_of_pair_sums(system, tip):
+    """The grid is no further from FP64 than the FP32 sum over every pair, which
+    the kernel of sheared cells gives for the same points (a shear of 1e-30): root
+    mean square of |dF| and of dE over boxes without near atoms, the dz2 tip
+    by its own stencil force.  Rounding alone differs, so 5 % are allowed."""
+    n, L = (32, 32, 32), [3.2, 3.2, 3.2]
+    xyz = {"molecule": lambda: M.molecule(60, 3)[0] * [1, 1, 1] + [1.6, 1.6, -7.5], "ring": lambda: _shell(200, L, 6.2, 12.0, 4),
+           "slab": lambda: _slab(-9.0, 70.0, 3000), "far slab": lambda: _slab(-33.0, 90.0, 3000)}[system]()
+    rng = np.random.default_rng(2)
+    Zs = np.full(len(xyz), 79) if "slab" in system else rng.choice([1, 6, 7, 8], len(xyz))
+    qs = np.zeros(len(xyz)) if "slab" in system else rng.uniform(-0.3, 0.3, len(xyz))
+    if "slab" in system:
+        qs[::40] = 0.1
+    cLJs = C.REA2LJ(C.getAtomsREA(8, Zs, C.loadSpecies(), alphaFac=-1.0))
+    xyzq = np.concatenate([xyz, qs[:, None]], 1)
+    model = D.ff_model(1, with_lj=True, stencil=list(zip(*tip)), with_energy=True, fmax=None)
+    FE = O.ljc_qzs_ff(n, np.array([[0, 0, 0], *np.diag(L)]), xyzq, cLJs, *tip)
+    e = []
+    for shear in (0.0, 1e-30):
+        cell = np.diag(L)
+        cell[0, 1] = shear
+        d = D.ff_build(n, cell, xyzq, cLJs, model, f64=False).download() - FE
+        e.append((np.sqrt((d[..., :3] ** 2).sum(-1).mean()), np.sqrt((d[..., 3] ** 2).mean())))
+    F, E = np.sqrt((FE[..., :3] ** 2).sum(-1).mean()), np.sqrt((FE[..., 3] ** 2).mean())
+    print(f"{system}: force {e[0][0] / F:.2e} pairs {e[1][0] / F:.2e}, energy {e[0][1] / E:.2e} pairs {e[1][1] / E:.2e}")
+    assert e[0][0] <= 1.05 * e[1][0]
+    assert e[0][1] <= 1.05 * e[1][1]
