@@ -307,7 +307,10 @@ constexpr double kVeryFarRatio = 40.0;
 constexpr int kGroups = 10;  // lane groups of kP2^2 that share the atoms, kP2 nodes along z a lane
 // Far atoms a box needs before the polynomial (56 FP64 FMAs per point) costs
 // less than their pair sums; below it every atom of the box counts as near.
-constexpr int kFarMin = 12;
+// 256x256x192 points, all near against far ones at the nodes: dz2 tip, 12 atoms
+// 238 and 123 us; one Coulomb point, 12 atoms 84 and 89, 20 atoms 123 and 100.
+template <int NS, bool Z0>
+constexpr int kFarMin = NS == 0 || (NS == 1 && Z0) ? 16 : 12;
 constexpr int kNodeFold = 8;  // FP32 partial-sum length at the nodes
 constexpr int kBoxTile = kThreads;  // atoms per LDS tile, one per thread
 constexpr int kNearCap = 512;       // near atoms listed; beyond, every atom is staged for each slab
@@ -343,7 +346,7 @@ struct BoxLds {
 
 template <bool LJ, int NS, bool Z0, bool WE, bool SEP>
 __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, const AtomRec *__restrict__ atoms,
-                                        float4 *__restrict__ out, int b)
+                                        float4 *__restrict__ out, int b, int slab0, int slab1)
 {
     constexpr int NG = WE ? 4 : 3;
     constexpr int G = SEP ? 2 : 1;
@@ -354,6 +357,7 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
     const int bz = b % A.nbz; b /= A.nbz;
     const int by = b % A.nby;
     const int bx = b / A.nby;
+    if (bx * kBox + slab0 * 4 >= A.n[0]) return;  // uniform
     const double dcx = A.dcell[0], dcy = A.dcell[4], dcz = A.dcell[8];
     constexpr double half = 0.5 * (kBox - 1);
     const double cx = bx * kBox + half, cy = by * kBox + half, cz = bz * kBox + half;
@@ -418,7 +422,7 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
                 nnear += L.count[1][q];
             }
             const unsigned long long below = (1ull << lane) - 1;
-            if (A.natoms <= kBoxTile && nf < kFarMin) {  // uniform: too few far atoms
+            if (A.natoms <= kBoxTile && nf < kFarMin<NS, Z0>) {  // uniform: too few far atoms
                 use_far = false;
                 nnear = A.natoms;
                 if (in && t < kNearCap) L.list[t] = t;
@@ -546,7 +550,7 @@ __device__ __forceinline__ void box_f32(const FFArgs &A, const FarTable &F, cons
     const double wcy = by * kBox + wave * 4 + 1.5, wcz = (bz * kBox / kZBrick) * kZBrick + 0.5 * (kZBrick - 1);
     const double fy = iy - wcy;
     const double oy = dcy * wcy, oz = dcz * wcz;
-    for (int slab = 0; slab < kBox / 4; slab++) {
+    for (int slab = slab0; slab < slab1; slab++) {
         if (bx * kBox + slab * 4 >= A.n[0]) break;  // uniform
         const int ix = bx * kBox + slab * 4 + xi;
         const double wcx = bx * kBox + slab * 4 + 1.5;
@@ -673,16 +677,18 @@ __host__ __device__ inline void set_boxes(FFArgs &A)
     A.nbz = (A.n[2] + kBox - 1) / kBox;
 }
 
-// One grid (items == nullptr) or every grid of a batch.  Three workgroups per
-// CU: LDS (46 KB) allows no more, so the registers need not either.
+// One grid (items == nullptr) or every grid of a batch; split: blocks per box
+// (box_split).  Three workgroups per CU: LDS (46 KB) allows no more, so the
+// registers need not either.
 template <bool LJ, int NS, bool Z0, bool WE, bool SEP>
 __global__ __launch_bounds__(kThreads, SEP ? 2 : 3) void ff_box_kernel(FFArgs A, FarTable F,
                                                                        const BatchGridItem *__restrict__ items,
                                                                        const long long *__restrict__ prefix, int nitems,
                                                                        const AtomRec *__restrict__ atoms,
-                                                                       float4 *__restrict__ out)
+                                                                       float4 *__restrict__ out, int split)
 {
-    long long b = blockIdx.x;
+    long long b = blockIdx.x / split;
+    const int slabs = kBox / 4 / split, slab0 = (blockIdx.x % split) * slabs;
     if (items) {
         const int m = find_item(prefix, nitems, b);
         const BatchGridItem it = items[m];
@@ -692,7 +698,7 @@ __global__ __launch_bounds__(kThreads, SEP ? 2 : 3) void ff_box_kernel(FFArgs A,
         atoms += it.atom_off;
         out += it.grid_off;
     }
-    box_f32<LJ, NS, Z0, WE, SEP>(A, F, atoms, out, (int)b);
+    box_f32<LJ, NS, Z0, WE, SEP>(A, F, atoms, out, (int)b, slab0, slab0 + slabs);
 }
 
 // Chebyshev points of the first kind, divided by the largest (which leaves
@@ -733,6 +739,24 @@ const FarTable &far_table()
     return F;
 }
 
+// Blocks per box.  A block takes as long on any grid (40 atoms, dz2 tip: 95 us),
+// so a launch that leaves CUs without work gives the four slabs of a
+// box to 2 or 4 blocks, each of which sums the nodes for itself; the points'
+// sums are the same.  1 / 2 / 4 blocks a box and, before boxes, the 4x4x64 bricks
+// over all atoms, us (dz2 tip, 40 atoms; one Coulomb point, 120 atoms):
+//   64 boxes    95 / 50 / 27, bricks 25     65 / 38 / 25, 27
+//   128         96 / 50 / 40, 40            65 / 38 / 31, 34
+//   175         96 / 58 / 49, 71            65 / 41 / 37, 58
+//   216         97 / 58 / 58, 88            66 / 43 / 50, 69
+//   392         125 / 94 / 95, 88           76 / 67 / 79, 71
+//   512         131 / 116 / 118, 138        78 / 81 / 92, 104
+//   768         115 / 121 / 140, 201        80 / 93 / 120, 149
+int box_split(unsigned boxes)
+{
+    constexpr unsigned cus = 256;
+    return boxes <= cus * 3 / 4 ? 4 : boxes <= cus * 7 / 4 ? 2 : 1;
+}
+
 template <bool LJ, int NS, bool Z0, bool WE, bool SEP>
 void launch_o(const FFArgs &A0, bool ortho, const AtomRec *atoms, void *out, const BatchLaunch *b, hipStream_t st)
 {
@@ -741,8 +765,10 @@ void launch_o(const FFArgs &A0, bool ortho, const AtomRec *atoms, void *out, con
     if (ortho) set_boxes(A);
     dim3 grid(b ? (unsigned)b->nbricks : (unsigned)A.nbx * A.nby * A.nbz);
     if (ortho) {
+        const int split = box_split(grid.x);
+        grid.x *= split;
         hipLaunchKernelGGL((ff_box_kernel<LJ, NS, Z0, WE, SEP>), grid, block, 0, st, A, far_table(), b ? b->items : nullptr,
-                           b ? b->prefix : nullptr, b ? b->nitems : 0, atoms, (float4 *)out);
+                           b ? b->prefix : nullptr, b ? b->nitems : 0, atoms, (float4 *)out, split);
     } else if (b) {
         if (LJ && NS > 0 && b->qskip)
             hipLaunchKernelGGL((ff_f32_batch_kernel<LJ, NS, Z0, WE, (LJ && NS > 0), SEP>), grid, block, 0, st, A, b->items,

@@ -2,7 +2,7 @@
 8 half widths summed at 8^3 Chebyshev nodes, beyond 40 half widths at 5^3
 (ff_grid_f32.hip box_f32), against
 the FP64 oracle where that split can go wrong: too few far atoms for the
-polynomial (11) and just enough (12), one LDS tile of 256 atoms and one more,
+polynomial (11, with one Coulomb point 15) and just enough (12, 16), one LDS tile of 256 atoms and one more,
 no far atom and no near atom at all, more near atoms than a box lists (512),
 partial boxes, unequal steps, both models and stencils, uncharged atoms, an
 atom that is not finite.
@@ -82,6 +82,8 @@ def _check(G, FE, bound):
 CASES = [
     ("11 far atoms", (16, 16, 16), (0.1, 0.1, 0.1), 3, 11),
     ("12 far atoms", (16, 16, 16), (0.1, 0.1, 0.1), 3, 12),
+    ("15 far atoms", (16, 16, 16), (0.1, 0.1, 0.1), 3, 15),
+    ("16 far atoms", (16, 16, 16), (0.1, 0.1, 0.1), 3, 16),
     ("no near atom", (33, 17, 31), (0.1, 0.1, 0.1), 0, 60),
     ("256 atoms", (20, 35, 18), (0.1, 0.1, 0.1), 6, 250),
     ("257 atoms", (20, 35, 18), (0.1, 0.1, 0.1), 6, 251),
@@ -288,3 +290,25 @@ def test_error_no_larger_than_of_pair_sums(system, tip):
     print(f"{system}: force {e[0][0] / F:.2e} pairs {e[1][0] / F:.2e}, energy {e[0][1] / E:.2e} pairs {e[1][1] / E:.2e}")
     assert e[0][0] <= 1.05 * e[1][0]
     assert e[0][1] <= 1.05 * e[1][1]
+
+
+@pytest.mark.parametrize("items", [1, 8, 17])
+def test_batch_of_small_grids_equals_single_grids(items):
+    """A box's slabs in 4 blocks (27 boxes alone, and in a batch), in 2 (8 grids: 216 boxes) and in one (17: 459)
+    give the same bits, over partial boxes and slabs too."""
+    n, L = (37, 40, 47), np.array([3.7, 4.0, 4.7])
+    lvec = np.array([[-2.0, -2.0, 3.0], [L[0], 0, 0], [0, L[1], 0], [0, 0, L[2]]])
+    mols = []
+    for k in range(items):
+        rng = np.random.default_rng(k)
+        m = (3, 40, 290)[k % 3]
+        mols.append((_shell(m, L, 3.0, 25.0, 20 + k) + lvec[0], rng.choice([1, 6, 8], m), rng.uniform(-0.2, 0.2, m)))
+    b = B.BatchScan.tilted([lvec] * items, [n] * items, pos0s=[(0.0, 0.0, 7.0)] * items, start=(-1, -1), end=(1, 1), scan_n=(8, 8),
+                           nz=10, molecules=mols, grid_f64=False)
+    b.run_stages(1)
+    b.synchronize()
+    for k, (xyz, Zs, qs) in enumerate(mols):
+        cLJs = C.REA2LJ(C.getAtomsREA(8, Zs, C.loadSpecies(), alphaFac=-1.0))
+        G = D.ff_build(n, lvec[1:], np.concatenate([xyz - lvec[0], qs[:, None]], 1), cLJs, b.model, f64=False).download()
+        assert np.array_equal(b.grid(k), G), k
+    b.close()
