@@ -350,14 +350,30 @@ constexpr int stage_batch()
     return WARM ? 4 : 1;
 }
 
+// Uniform values that every pass of a mode 1 column reads, in vector registers
+// (a single scan has registers to spare).  The kernel's uniform values exceed
+// the scalar registers, and the compiler then keeps some in lanes of a vector
+// register and reads them back one by one (v_readlane): 64 to 128 of a pass's 350
+// instructions; scans of 60 atoms: 64x64x30 0.99 ms with them, 0.81 without,
+// 192x192x30 1.17 and 0.94, 320x320x30 1.43 and 1.09.
+__device__ __forceinline__ void in_vgprs(DevArgs &A)
+{
+    for (double *p : {&A.conv_f2, &A.dtmax, &A.a0, &A.finc, &A.fdec, &A.falpha, &A.dtmin, &A.f2safe}) asm("" : "+v"(*p));
+    for (int k = 0; k < 9; k++) asm("" : "+v"(A.rot[k]));
+}
+
 // A wave relaxes a tile of A.tile_x x A.tile_y columns (64 or fewer, its
-// remaining lanes idle), or that many consecutive ones (A.tiles_y 0).  Block b runs its waves' consecutive tiles of part
-// b % 8 (one contiguous part of the tiles per XCD).
+// remaining lanes idle), or that many consecutive ones (A.tiles_y 0).  Block b
+// runs its waves' consecutive tiles of part b % 8 (one contiguous part of the
+// tiles per XCD).  Records are staged for 64 lanes whatever the tile: slots
+// counted by the tile cost scalar registers (192x192x30 scan in mode 1 1.17 ms, 1.06
+// with 64).
 // FRAC 0 in tiles of a few columns, where lanes seldom wait together.
 template <typename T4, int MODE, bool ORTHO, int WPB, int FRAC>
 __global__ __launch_bounds__(64 * WPB) void relax_dev_kernel(DevArgs A, const T4 *__restrict__ grid)
 {
-    extern __shared__ __align__(16) unsigned char single_lds[];  // kStageSingle records per column
+    __shared__ __align__(16) unsigned char lds[kStageSingle * 64 * WPB * kStageRecordBytes];
+    Stage<kStageSingle> G = make_stage<kStageSingle>(lds, 64 * WPB, threadIdx.x);
     const int wave = WPB == 1 ? 0 : (int)(threadIdx.x / 64);
     const int lane = WPB == 1 ? (int)threadIdx.x : (int)(threadIdx.x % 64);
     const int cols = A.tile_x * A.tile_y;
@@ -365,7 +381,6 @@ __global__ __launch_bounds__(64 * WPB) void relax_dev_kernel(DevArgs A, const T4
     const int b = blockIdx.x;
     const int tile = ((b % 8) * per_xcd + b / 8) * WPB + wave;
     if (tile >= A.ntiles) return;
-    Stage<kStageSingle> G = make_stage<kStageSingle>(single_lds, cols * WPB, wave * cols + min(lane, cols - 1));
     int i, j;
     if (A.tiles_y > 0) {
         const int ti = tile / A.tiles_y, tj = tile % A.tiles_y;
@@ -376,6 +391,7 @@ __global__ __launch_bounds__(64 * WPB) void relax_dev_kernel(DevArgs A, const T4
         i = c / A.ny;
         j = c - i * A.ny;
     }
+    if (MODE == 1) in_vgprs(A);
     unsigned long long nevals = 0, npos = 0;
     unsigned turns = 0;
     relax_column<T4, MODE, kStageSingle, ORTHO, FRAC>(A, grid, i, j, lane < cols && i < A.nx && j < A.ny, G, nevals, npos, turns);
@@ -612,8 +628,7 @@ template <typename T4, int MODE, bool ORTHO, int WPB, int FRAC>
 static void launch_single_w(const DevArgs &A, const void *grid, hipStream_t st)
 {
     const long nb = (((A.ntiles + WPB - 1L) / WPB + 7) / 8) * 8;
-    const size_t lds = (size_t)A.tile_x * A.tile_y * WPB * kStageSingle * kStageRecordBytes;
-    hipLaunchKernelGGL((relax_dev_kernel<T4, MODE, ORTHO, WPB, FRAC>), dim3((unsigned)nb), dim3(64 * WPB), lds, st, A,
+    hipLaunchKernelGGL((relax_dev_kernel<T4, MODE, ORTHO, WPB, FRAC>), dim3((unsigned)nb), dim3(64 * WPB), 0, st, A,
                        (const T4 *)grid);
 }
 
