@@ -334,8 +334,10 @@ class BatchScan:
 
     def lane_use(self):
         """Force evaluations of the last relaxation over its lane slots (64 per
-        loop pass of each wave): the fraction of SIMD lanes that did work while
-        a wave waited for its slowest column."""
+        loop pass of each wave): the fraction of slots in which a lane evaluated
+        a force.  The others are those of lanes whose column had ended while the
+        wave's slowest had not, and those in which a running lane waited to load
+        its cell or store its record together with others, by design."""
         c = np.empty(4, np.uint64)
         check(lib().ppafm_memcpy_d2h(c.ctypes.data, lib().ppafm_batch_buffer(self._h, BUF_COUNTERS), 32, self.stream), "download")
         return float(c[0]) / float(c[3]) if c[3] else float("nan")

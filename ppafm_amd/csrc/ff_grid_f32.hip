@@ -1,6 +1,6 @@
 // FP32 force-field grid kernel on gfx950 (the float4 grid of the OpenCL
 // path, FF.cl:366-423 evalLJC_QZs_noPos, and an FP32 variant of the
-// ProbeParticle grid, Forces.h:120-132 / 237-244): VALU bound.
+// ProbeParticle grid, Forces.h:120-132 / 237-244): bound by VALU issue.
 //
 //   * Orthogonal cells: boxes of 16^3 points with the far atoms on Chebyshev
 //     nodes (box_f32).  Sheared cells: brick mapping as the FP64 kernel (4x4
@@ -278,8 +278,11 @@ __device__ __forceinline__ void brick_f32(const FFArgs &A, const AtomRec *__rest
 // nearer are summed at every point.  A far pair costs 1/8 of a near one.  With
 // more atoms than one LDS tile, those beyond kVeryFarRatio half widths are
 // summed at kP2^3 nodes (1/33), whose polynomial is added to the values at the
-// kP^3 nodes.  VALU bound as before, in the near pairs for a molecule, in the
-// nodes for a slab.
+// kP^3 nodes.  Bound by VALU issue, in the near pairs for a molecule, in the
+// nodes for a slab: of a wave's time 53 % is issue (slab; 49 % molecule), 30 %
+// (35 %) waiting for a slot that another wave holds, 17 % (16 %) for loads, LDS
+// and barriers, 0.04 % (0.5 %) LDS bank conflicts; 2.8 (2.3) waves on a SIMD, a
+// VALU instruction every 3.1 (4.4) cycles.
 // Interpolation error at 0.1 A steps, against the far atom's own force at the
 // point, largest over a box that faces the atom (an atom off its edges or
 // corners: a tenth), in FP64: order 8 at ratio 8 (6 A) 5.9e-7 for H, 4.1e-7 O,
@@ -295,9 +298,9 @@ __device__ __forceinline__ void brick_f32(const FFArgs &A, const AtomRec *__rest
 // changes it was 1.02 and 1.08, 1.18 and 1.17.  Node coordinates are FP32 while
 // the weights assume exact nodes: 3e-8 A at 0.75 A, 4e-8 of the force at 6 A.
 // Measured (grid kernel, before: every atom at every point): 60 atoms, dz2
-// tip, 256x256x192 points 1277 -> 373 us; 16 such grids of 8-120 atoms
-// 23.5 -> 6.6 ms; 17,928 atoms, 400x400x300 points 321 -> 43 ms with one set of
-// nodes, 15.3 ms with two.
+// tip, 256x256x192 points 1254 -> 368 us; 16 such grids of 8-120 atoms
+// 24.1 -> 6.8 ms; 17,928 atoms, 400x400x300 points 319 -> 43 ms with one set of
+// nodes, 15.4 ms with two.
 constexpr int kBox = 16;
 constexpr int kP = 8;
 constexpr double kFarRatio = 8.0;

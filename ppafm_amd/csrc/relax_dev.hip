@@ -14,8 +14,6 @@
 // Lanes run independent state machines over (z step, iteration) and stage
 // their output records in LDS (Stage, relax_dev.hpp).
 
-#include <cstdlib>
-
 #include "pp_common.hpp"
 
 #pragma clang fp contract(off)
@@ -90,10 +88,14 @@ __device__ __forceinline__ void column_init(const DevArgs &A, Column<NC> &C, int
 
 // Shares of a wave's running lanes that wait before it turns to them (serve):
 // plain FIRE, ProbeParticle and OpenCL semantics, and warm starts.  Measured
-// from one lane (at once) down to half the wave: 256x256x60 scan 8.8 ms at
+// from one lane (at once) up to half the wave: 256x256x60 scan 8.8 ms at
 // once, 6.6 at 1/16, 6.4 at 1/8, 7.2 at 1/4; 48 molecules of 128x128x30 plain
-// 16.1, 13.1, 12.9, 16.9; Newton 6.4 ms at once, 5.6 at 1/8, 5.2 at 1/4, 5.1
-// at 1/2; 400x400x60 tilted scan 3.3, 2.7, 2.6, 2.8.
+// 16.1, 13.1, 12.9, 16.9; OpenCL semantics, in batches: 16 images of
+// 128x128x30 1.89 ms at once, 1.67 at 1/16, 1.51 at 1/8, 1.48 at 1/4, a
+// 400x400x60 tilted scan 3.58, 3.13, 2.97, 2.74; Newton 6.4 ms at once, 5.6 at
+// 1/8, 5.2 at 1/4, 5.1 at 1/2 (other molecules: 8.2 ms without waiting lanes and
+// the polynomial, 7.7 with both; the whole call of the batch, FP64 grid included,
+// 16.1 and 15.5).
 constexpr int kServe[2] = {8, 4};
 constexpr int kServeWarm = 4;
 
@@ -588,8 +590,6 @@ __global__ __launch_bounds__(256) void relax_refill_kernel(DevArgs A, BatchArgs 
 
 }  // namespace
 
-// 0 on launch, 1 when the parameters need the generic kernel (leap-frog,
-// max_iters < 1), negative on error.
 // SIMDs of the current device (4 per CU), 0 if unknown
 static int simd_count()
 {
@@ -657,6 +657,8 @@ static void launch_single(const DevArgs &A0, const void *grid, hipStream_t st)
     else launch_single_w<T4, MODE, ORTHO, 1, 0>(A, grid, st);
 }
 
+// 0 on launch, 1 when the parameters need the generic kernel (leap-frog,
+// max_iters < 1), negative on error.
 int launch_relax_fast(const RelaxLaunch &L, const void *grid, bool f64, hipStream_t st)
 {
     if (L.rp.alg != 1 || L.rp.max_iters < 1) return 1;

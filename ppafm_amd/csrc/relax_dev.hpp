@@ -1,7 +1,9 @@
 // Device helpers of the FIRE relaxation shared by relax_dev.hip and
 // ws_batch.hip: kernel arguments, periodic trilinear sampling (Grid.h:66-69
 // semantics), the tip springs and one FIRE move.  Contraction is off in the
-// files that include this, so every kernel rounds identically.
+// files that include this, so kernels that share a function round identically.
+// Columns sample a cell's polynomial (CellCache), fire_points_kernel the
+// weighted corners (gather): the same field, rounded differently.
 #pragma once
 
 #include "pp_common.hpp"

@@ -427,6 +427,8 @@ __global__ __launch_bounds__(64) void ws_bwd1b_kernel(long K, int kr, const unsi
             }
 }
 
+// Adam on the FP32 master parameters; refreshes the bf16 copies and clears
+// the gradient.  step >= 1.
 __global__ __launch_bounds__(256) void ws_adam_kernel(float *__restrict__ theta, float *__restrict__ grad,
                                                       float *__restrict__ m1, float *__restrict__ m2, float lr,
                                                       float beta1, float beta2, float eps, float c1, float c2,
