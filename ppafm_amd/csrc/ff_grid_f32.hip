@@ -754,9 +754,13 @@ const FarTable &far_table()
 //   392         125 / 94 / 95, 88           76 / 67 / 79, 71
 //   512         131 / 116 / 118, 138        78 / 81 / 92, 104
 //   768         115 / 121 / 140, 201        80 / 93 / 120, 149
-int box_split(unsigned boxes)
+// With more than one tile of atoms, both sets of nodes and twice the passes over
+// the atoms are repeated, and it pays up to half as many boxes only (400 atoms,
+// dz2 tip): 64 boxes 243 / 174 / 140, 128 244 / 174 / 206, 216 263 / 230 / 359,
+// 392 346 / 400 / 615.  (A batch's atoms are not known here.)
+int box_split(unsigned boxes, bool two_sets)
 {
-    constexpr unsigned cus = 256;
+    const unsigned cus = two_sets ? 128 : 256;
     return boxes <= cus * 3 / 4 ? 4 : boxes <= cus * 7 / 4 ? 2 : 1;
 }
 
@@ -768,7 +772,7 @@ void launch_o(const FFArgs &A0, bool ortho, const AtomRec *atoms, void *out, con
     if (ortho) set_boxes(A);
     dim3 grid(b ? (unsigned)b->nbricks : (unsigned)A.nbx * A.nby * A.nbz);
     if (ortho) {
-        const int split = box_split(grid.x);
+        const int split = box_split(grid.x, !b && A.natoms > kBoxTile);
         grid.x *= split;
         hipLaunchKernelGGL((ff_box_kernel<LJ, NS, Z0, WE, SEP>), grid, block, 0, st, A, far_table(), b ? b->items : nullptr,
                            b ? b->prefix : nullptr, b ? b->nitems : 0, atoms, (float4 *)out, split);
